@@ -1258,6 +1258,12 @@ p2k::GemmArgs gemm_args(int M, int N, int K, float alpha, float beta, const sign
     return g;
 }
 
+/* the plan runs on gemm_fv_rb */
+bool records_in_regs(const Plan &p, int mode)
+{
+    return (p.cfg == FV_W6 || p.cfg == FV_WK) && mode != P2H_INT8 && switch_of(g_sw.records_in_regs) != 0;
+}
+
 /* the large-M tiles: unsplit, two workgroups per CU, 4-bit records (in registers, or through the LDS ring with the
  * activation rows), staged output rows */
 template <class G>
@@ -1265,8 +1271,11 @@ void launch_fv_large(const p2k::GemmArgs &g, const Plan &p, hipStream_t s)
 {
     const dim3 grid((unsigned)((size_t)p.tiles_m * p.tiles_n)), block(G::NT);
     if (switch_of(g_sw.records_in_regs)) {
-        if (g.K > p2k::kFoldRows) hipLaunchKernelGGL((p2k::gemm_fv_rb<G, true>), grid, block, 0, s, g);
-        else hipLaunchKernelGGL((p2k::gemm_fv_rb<G, false>), grid, block, 0, s, g);
+        const bool multi = g.K > p2k::kFoldRows;
+        if (multi && g.act) hipLaunchKernelGGL((p2k::gemm_fv_rb<G, true, true>), grid, block, 0, s, g);
+        else if (multi) hipLaunchKernelGGL((p2k::gemm_fv_rb<G, true, false>), grid, block, 0, s, g);
+        else if (g.act) hipLaunchKernelGGL((p2k::gemm_fv_rb<G, false, true>), grid, block, 0, s, g);
+        else hipLaunchKernelGGL((p2k::gemm_fv_rb<G, false, false>), grid, block, 0, s, g);
         return;
     }
     if (g.K > p2k::kFoldRows)
@@ -1350,8 +1359,7 @@ const char *p2h_fvb_plan(int mode, int M, int N, int K, int with_workspace)
         snprintf(buf, sizeof buf, "tile %dx%d, %d split%s of %d rows%s%s", kFvBM[p.cfg], kFvBN[p.cfg], p.splits,
                  p.splits > 1 ? "s" : "", p.split_rows,
                  p.splits > 1 ? " + fold" : (K > p2k::kFoldRows ? ", folds in registers" : ""),
-                 (p.cfg == FV_W6 || p.cfg == FV_WK) && mode != P2H_INT8 && switch_of(g_sw.records_in_regs)
-                     ? ", weight records in registers" : "");
+                 records_in_regs(p, mode) ? ", weight records in registers" : "");
     return buf;
 }
 
@@ -1391,7 +1399,8 @@ int p2h_fvb_gemm_q8a_silu(int mode, int M, int N, int K, float alpha, const sign
 }
 
 /* silu: C = silu_p2(alpha·A·W) with beta 0, ldc = N and N % 8 == 0 (p2_swish over whole rows: every element in
- * the eight-wide body); small-M tiles apply it in their epilogue, the others by p2h_silu after the GEMM. */
+ * the eight-wide body); gemm_fvs and gemm_fv_rb apply it in their epilogues (the latter 42 µs of a second pass less
+ * at M = 6000, N = 4096), the other tiles by p2h_silu after the GEMM. */
 static int fvb_gemm_q8a(int mode, int M, int N, int K, float alpha, const signed char *dQ, int ldq,
                         const float *dScales, const P2hWeight *w, float beta, float *dC, int ldc, void *workspace,
                         size_t workspace_bytes, const P2hWeight *next, void *stream, bool silu)
@@ -1421,7 +1430,7 @@ static int fvb_gemm_q8a(int mode, int M, int N, int K, float alpha, const signed
         g.warm = next->rec4;
         g.warm_lines = (int)std::min<size_t>((bytes + 127) / 128, 0x7fffffff);
     }
-    const bool silu_here = silu && is_small(p.cfg);
+    const bool silu_here = silu && (is_small(p.cfg) || records_in_regs(p, mode));
     g.act = silu_here ? 1 : 0;
     if (mode == P2H_INT8W) {
         g.c1 = w->hi; g.c1_hi = 1;

@@ -1300,7 +1300,7 @@ struct GemmArgs {
     int kst;                                              /* 64-column steps per 16-row group of Q: ldq / 64 */
     int mg_last, ng_last;                                 /* last 16-row group of Q, last 16-column group of C */
     const uint8_t *warm; int warm_lines;                  /* 128-byte lines a later kernel reads, loaded meanwhile */
-    int act;                                              /* small-M tiles: 1 stores silu_p2 of each output */
+    int act;                                              /* 1: silu_p2 of each output (gemm_fvs, gemm_fv_rb) */
     int xcd_rows;                                         /* small-M tiles: 0, or the rows of an XCD grid (below) */
 };
 
@@ -2162,7 +2162,7 @@ __device__ __forceinline__ void fv_tile(const GemmArgs &g)
  *  barrier per stage). Against the records in LDS: M = 1500 11.3 against 12.4 µs, M = 4099 24.8 against 27.1,
  *  M = 6000 32.5 against 33.7 (1024 → 4096). Two workgroups per CU; the output is folded and staged as in
  *  fv_tile (per 1024-row block, in order; C staged through LDS as whole row segments at device scope). */
-template <class G, bool MULTI>
+template <class G, bool MULTI, bool ACT>
 __device__ __forceinline__ void fv_tile_rb(const GemmArgs &g)
 {
     constexpr int FM = G::FM, FN = G::FN, NW = G::NW, D = G::D, A_STAGE = G::A_STAGE, A_DMA = G::A_DMA;
@@ -2378,7 +2378,11 @@ __device__ __forceinline__ void fv_tile_rb(const GemmArgs &g)
         for (int r = wave * RPI + lr; r < rows; r += NW * RPI) {
             const int m = m0 + 16 * j0 + r, n = n0 + 4 * lc;
             if (m < M && n < N) {
-                const v4f v = *reinterpret_cast<const v4f *>(stg + r * SROW + 4 * lc);
+                v4f v = *reinterpret_cast<const v4f *>(stg + r * SROW + 4 * lc);
+                if (ACT) {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) v[e] = silu_p2(v[e]);
+                }
                 if (g.c_vec4) {
                     cout.st16(((size_t)(m - m0) * g.ldc + n) * 4, v);
                 } else {
@@ -2391,10 +2395,14 @@ __device__ __forceinline__ void fv_tile_rb(const GemmArgs &g)
     }
 }
 
-template <class G, bool MULTI>
+/* ACT: silu_p2 of each finished output (GemmArgs::act), the feed-forward's SiLU as fvs_tile applies it, on the row
+ * segments between the staging and the store. As a pass of its own after the GEMM it reads and writes C again:
+ * 42 µs at M = 6000, 1024 → 4096, beside the GEMM's 33; here it costs 7 of them (the feed-forward half step at 6000
+ * rows 160.3 → 125.1 µs). */
+template <class G, bool MULTI, bool ACT>
 __global__ __launch_bounds__(G::NT, 2) void gemm_fv_rb(GemmArgs g)
 {
-    fv_tile_rb<G, MULTI>(g);
+    fv_tile_rb<G, MULTI, ACT>(g);
 }
 
 template <class G, int MODE, int OUT, bool MULTI, bool SPLIT, int OCC = 1, bool CSHUF = false>

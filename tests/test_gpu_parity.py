@@ -366,13 +366,28 @@ def test_q8a_next_matches_q8a(mode, M, K, N, Kn, Nn, beta):
 @pytest.mark.parametrize("mode", ["int8w", "int8"])
 @pytest.mark.parametrize("M,K,N", [(375, 1024, 4096), (38, 1024, 4096), (375, 4096, 272), (2000, 1024, 1024)])
 def test_q8a_silu_matches_gemm_then_silu(mode, M, K, N):
-    """p2h_fvb_gemm_q8a_silu equals p2h_fvb_gemm_q8a followed by p2h_silu bit for bit: the small-M tiles apply
-    silu_p2 as they store C; at 2000 rows (the large-M kernel) the library runs the SiLU kernel after the GEMM."""
+    """p2h_fvb_gemm_q8a_silu equals p2h_fvb_gemm_q8a followed by p2h_silu bit for bit: the small-M tiles and the
+    int8w large-M tiles apply silu_p2 as they store C; the two-plane mode at 2000 rows runs the SiLU kernel after
+    the GEMM."""
     A = P.gen_activations(SEED, 1900 + M, M, K)
     q, sc = O.quant_rows(A)
     w = P.FvWeight(*_weight(K, N, 1910 + N), K, N)
     got = P.fvb_gemm_q8a_silu(mode, q, sc, w, alpha=0.7)
     ref = P.silu(P.fvb_gemm_q8a(mode, q, sc, w, alpha=0.7))
+    assert np.isfinite(got).all()
+    assert _bits_equal(got, ref)
+
+
+@pytest.mark.parametrize("M,K,N", [(2101, 128, 4112), (1025, 1024, 272), (1030, 1156, 16), (1100, 4096, 144)])
+def test_q8a_silu_large_tiles(M, K, N):
+    """The int8w large-M tiles' SiLU (96 x 256 and 96 x 128, one and several fold blocks) with a cut last row tile and
+    column tile: the bits of the GEMM followed by p2h_silu."""
+    print(f"q8a silu large M={M} K={K} N={N} {P.plan('int8w', M, N, K)}", flush=True)
+    A = P.gen_activations(SEED, 1950 + M, M, K)
+    q, sc = O.quant_rows(A)
+    w = P.FvWeight(*_weight(K, N, 1960 + N), K, N)
+    got = P.fvb_gemm_q8a_silu("int8w", q, sc, w, alpha=0.7)
+    ref = P.silu(P.fvb_gemm_q8a("int8w", q, sc, w, alpha=0.7))
     assert np.isfinite(got).all()
     assert _bits_equal(got, ref)
 
