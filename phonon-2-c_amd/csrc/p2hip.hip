@@ -16,6 +16,7 @@
 #include <mutex>
 
 #include "p2hip_kernels.h"
+#include "p2hip_split.h"
 
 namespace {
 
@@ -201,6 +202,7 @@ struct P2hWeight {
     uint8_t *rec4;    /* 4-bit selector records, the operand of every GEMM route (fv_repack4):
                          [N/16][units][64 lanes][16 B] */
     int units;        /* 128-row K units: K rounded up / 128 */
+    bool planes;      /* no code 3 and every lo and hi finite, below 2^100: the exact route's plane kernels take it */
     void *own;        /* the one device allocation this handle made */
     size_t own_bytes;
 };
@@ -491,12 +493,18 @@ static int weight_tables(P2hWeight *w)
     hipLaunchKernelGGL(p2k::fv_tables, dim3((w->N + 255) / 256), dim3(256), 0, s, w->N, w->lo, w->hi, w->clo);
     HIPCHK(hipGetLastError());
     const size_t recs = (size_t)(w->N / 16) * w->units * 64;
+    uint32_t odd = 0;   /* the word after the records: set by the kernels for what the plane kernels cannot hold */
     if (recs > 0) {
+        uint32_t *d_odd = (uint32_t *)(w->rec4 + recs * 16);
+        hipLaunchKernelGGL(p2k::fill_u32, dim3(1), dim3(256), 0, s, d_odd, (size_t)1, 0u);
         hipLaunchKernelGGL(p2k::fv_repack4, dim3((unsigned)((recs + 255) / 256)), dim3(256), 0, s, w->K, w->N,
-                           w->units, w->signs, w->flags, (uint4 *)w->rec4);
+                           w->units, w->signs, w->flags, (uint4 *)w->rec4, d_odd);
+        hipLaunchKernelGGL(p2k::fv_check, dim3((w->N + 255) / 256), dim3(256), 0, s, w->N, w->lo, w->hi, d_odd);
         HIPCHK(hipGetLastError());
+        HIPCHK(hipMemcpyAsync(&odd, d_odd, sizeof odd, hipMemcpyDeviceToHost, s));
     }
     HIPCHK(hipStreamSynchronize(s));
+    w->planes = odd == 0;
     return P2H_OK;
 }
 
@@ -1562,11 +1570,10 @@ static int launch_exact(int bkind, const p2k::ExactArgs &g0, hipStream_t s)
     return P2H_OK;
 }
 
-/* The exact five-value route on the fp32 matrix cores (gemm_xf): 32 × 64 tiles, or 32 × 32 where 32 × 64 would leave
- * fewer than two workgroups per CU; rows staged through LDS by direct loads where K % 128 == 0 and the rows allow
- * 16-byte loads (the same bits as the register path, which P2H_XF_STAGED=0 selects). P2H_EXACT_CHAIN=1 selects
- * gemm_exact instead, the reference's per-output fmaf chain bit for bit; P2H_XF_TILE = 32 or 64 forces the tile
- * width. */
+/* The exact five-value route on the matrix cores: gemm_xs for many rows, else gemm_xf (rows staged through LDS by
+ * direct loads where K % 128 == 0 and the rows allow 16-byte loads; the same bits as the register path, which
+ * P2H_XF_STAGED=0 selects). P2H_EXACT_CHAIN=1 selects gemm_exact instead, the reference's per-output fmaf chain bit for
+ * bit; P2H_XF_TILE forces gemm_xf and its tile. */
 }  // extern "C"
 
 namespace {
@@ -1582,19 +1589,31 @@ void launch_xf_tile(const p2k::ExactArgs &g, hipStream_t s)
     else hipLaunchKernelGGL((p2k::gemm_xf<FM, FN, false>), grid, block, 0, s, g);
 }
 
+using XsL = p2k::XsGeo<2, 2, 2, 4>;   /* 64 × 128 */
+
 int launch_xf(const p2k::ExactArgs &g0, hipStream_t s)
 {
     p2k::ExactArgs g = g0;
     const long long cus = g_cus > 0 ? g_cus : 256;
-    /* measured at M = 38 to 749 (the weights from HBM, the same bits for every tile): 16 × 16 tiles while they
-     * number at most six per CU (M = 38, 4096 -> 1024: 13.3 against 27.2 µs; M = 375, 4096 -> 1024: 41.4 against
-     * 44.9 µs), then 32 × 64 where those fill three workgroups per CU, else 32 × 32 (M = 375, 1024 -> 3072: 29.6
-     * against 33.3 µs for 32 × 64) */
-    const long long t16 = (long long)((g.N + 15) / 16) * ((g.M + 15) / 16);
-    const long long t64 = (long long)((g.N + 63) / 64) * ((g.M + 31) / 32);
-    int bm = t16 <= 6 * cus ? 16 : 32;
-    int bn = bm == 16 ? 16 : (t64 >= 3 * cus ? 64 : 32);
+    auto tiles = [&](int bm, int bn) { return (long long)((g.N + bn - 1) / bn) * ((g.M + bm - 1) / bm); };
     const int forced = switch_of(g_sw.xf_tile);
+    /* many rows: where gemm_xs' tiles fill its two workgroups per CU at least once (M = 6000, 1024 -> 4096: 228 against
+     * 272 µs for gemm_xf's best tile; at 192 tiles, M = 375, 28.4 against 21.9) */
+    if (forced == 0 && tiles(XsL::BM, XsL::BN) >= 2 * cus && g.K % 4 == 0 && g.K >= 64 && g.lda % 4 == 0 &&
+        aligned(g.A, 16)) {
+        g.tiles_n = (g.N + XsL::BN - 1) / XsL::BN;
+        const dim3 grid((unsigned)(8 * ((tiles(XsL::BM, XsL::BN) + 7) / 8))), block(XsL::NT);
+        if (g.K % 64 == 0) hipLaunchKernelGGL((p2k::gemm_xs<XsL, false>), grid, block, 0, s, g);
+        else hipLaunchKernelGGL((p2k::gemm_xs<XsL, true>), grid, block, 0, s, g);
+        HIPCHK(hipGetLastError());
+        return P2H_OK;
+    }
+    /* measured with the weights from HBM, the same bits for every tile: 16 × 16 while those fit the CUs in one round
+     * (M = 38, 4096 -> 1024: 10.7 against 11.4 µs for 16 × 32), 16 × 32 up to three per CU (M = 125, 1024 -> 1024: 5.4
+     * against 5.8 and 6.9 for 16 × 16 and 16 × 64; M = 375, 4096 -> 1024: 25.4 against 33.8 and 27.9), 16 × 64 up to
+     * six (M = 125, 1024 -> 4096: 9.9 against 10.7 and 10.1 for 16 × 32 and 32 × 64), else 32 × 64 */
+    int bm = 16, bn = tiles(16, 16) <= cus ? 16 : tiles(16, 32) <= 3 * cus ? 32 : 64;
+    if (bn == 64 && tiles(16, 64) > 6 * cus) bm = 32;
     if (forced == 32 || forced == 64) { bm = 32; bn = forced; }
     if (forced == 1616 || forced == 1632 || forced == 1664) { bm = 16; bn = forced - 1600; }
     g.tiles_n = (g.N + bn - 1) / bn;
@@ -1650,7 +1669,9 @@ static int exact_gemm(int M, int N, int K, float alpha, const float *dA, int lda
     g.lo = w->lo; g.hi = w->hi;
     g.C = dC; g.ldc = ldc;
     g.rec = w->rec4; g.units = w->units;
-    if (switch_of(g_sw.exact_chain) != 0 || K == 0) {
+    g.c_vec4 = ldc % 4 == 0 && aligned(dC, 16);
+    g.c_wt = switch_of(g_sw.dev_scope_stores) ? 1 : 0;
+    if (switch_of(g_sw.exact_chain) != 0 || K == 0 || !w->planes) {
         if (int rc = launch_exact(p2k::EXB_FV, g, s)) return rc;
         return silu ? p2h_silu((size_t)M * N, dC, s) : P2H_OK;
     }

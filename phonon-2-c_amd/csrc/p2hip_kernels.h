@@ -1782,7 +1782,7 @@ void gemm_i8(GemmArgs g)
  * brings a whole 128-row unit, and an operand dword decodes with one mask (and one shift for odd d) before the
  * table permute. */
 __global__ void fv_repack4(int K, int N, int units, const uint8_t *__restrict__ signs,
-                           const uint8_t *__restrict__ flags, uint4 *__restrict__ rec)
+                           const uint8_t *__restrict__ flags, uint4 *__restrict__ rec, uint32_t *__restrict__ odd)
 {
     const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= (size_t)(N / 16) * units * 64) return;
@@ -1791,6 +1791,7 @@ __global__ void fv_repack4(int K, int N, int units, const uint8_t *__restrict__ 
     const int u = (int)(gu % units), cg = (int)(gu / units);
     const int n = 16 * cg + (l & 15), kq = l >> 4;
     uint32_t w[4] = {0u, 0u, 0u, 0u};
+    bool any3 = false;
     for (int s = 0; s < 2; s++)
         for (int d = 0; d < 4; d++)
             for (int b = 0; b < 4; b++) {
@@ -1800,9 +1801,21 @@ __global__ void fv_repack4(int K, int N, int units, const uint8_t *__restrict__ 
                     code = (signs[(size_t)k * (N / 4) + (n >> 2)] >> (2 * (n & 3))) & 3u;
                     flag = (flags[(size_t)k * (N / 8) + (n >> 3)] >> (n & 7)) & 1u;
                 }
+                any3 |= code == 3u;
                 w[2 * s + (d >> 1)] |= (code | (flag << 2)) << (8 * b + 4 * (d & 1));
             }
+    if (any3) *odd = 1u;   /* code 3 (twice the value): the exact route's plane kernels cannot hold it */
     rec[idx] = make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+/* *odd = 1 where a column's lo or expanded hi is not finite or is 2^100 or more (the plane kernels scale their sums by
+ * both, used or not). */
+__global__ void fv_check(int N, const float *__restrict__ lo, const float *__restrict__ hi, uint32_t *__restrict__ odd)
+{
+    const int n = blockIdx.x * blockDim.x + threadIdx.x;
+    if (n >= N) return;
+    const float l = lo[n], h = __builtin_fmaf(1.0f, hi[n] - l, l), big = 1267650600228229401496703205376.0f;
+    if (!(__builtin_fabsf(l) < big && __builtin_fabsf(h) < big)) *odd = 1u;
 }
 
 /* The selector nibble (code | flag << 2, fv_repack4's layout) of weight (k, n) lives in record (n / 16, k / 128),
@@ -2746,7 +2759,8 @@ struct ExactArgs {
     const int8_t *B8; int ldb; const float *bscales;      /* int8 table */
     float *C; int ldc;
     int tiles_n;
-    const uint8_t *rec; int units;                        /* 4-bit selector records (fv_repack4) for gemm_xf */
+    const uint8_t *rec; int units;                        /* 4-bit selector records (fv_repack4) */
+    int c_vec4, c_wt;                                     /* gemm_xs: as in GemmArgs */
     int act;                                              /* gemm_xf: 1 stores silu_p2 of each output (beta 0,
                                                              ldc = N, N % 8 == 0: p2_swish's eight-wide body) */
 };
@@ -2886,21 +2900,104 @@ __global__ __launch_bounds__(256) void gemm_exact(ExactArgs g)
     }
 }
 
-/* The exact-mode five-value GEMM on the fp32 matrix cores (sgemm_fvb_exact, blas.c:929-987): C = beta·C +
- * alpha·A·W with every weight expanded to fp32 as the reference expands it, w = (code − 1)·fmaf(flag, hi − lo, lo)
- * (blas.c:875-897), and the products summed in fp32 by v_mfma_f32_16x16x4_f32. The sum runs in a different order
- * from the reference's per-output fmaf chain (which gemm_exact keeps bit for bit), so outputs agree to fp32 rounding.
+/* ── exact products on the bf16 matrix cores ───────────────────────────────────────────────────────────────────
+ * The exact route's products of fp32 rows with five-value weights, w = (code − 1)·v with v = lo or hi by the flag. A
+ * row's value is cut into three bf16 parts (8 + 8 + 8 significand bits, their sum exactly the value), and the weights
+ * into two planes of −1/2, 0, 1/2: the signs where the flag is clear and where it is set. Every product of a part with
+ * a plane is exact, the sums are fp32 as on the fp32 matrix cores, and 2·lo and 2·hi scale the two planes' sums at the
+ * end: six bf16 matrix instructions of 32 k against eight fp32 ones of 4 k for the same work, at a sixteenth of the
+ * time each. No value is rounded on the way in and a 32-k step rounds a sum three times instead of eight, so the
+ * outputs are nearer to the 64-bit ones than the fp32 instructions': 1.6e-7 against 2.3e-7 (relative, K = 1024) and
+ * 1.7e-7 against 4.5e-7 (K = 4096).
+ *   Rows holding a value of 2^112 or more (or an infinity, whose parts are not finite) are summed by a scalar chain
+ * of fmaf over the expanded weights instead (xs_big_row): the planes' zeros would make NaN of an infinity, and the
+ * halves could overflow where the real weights do not. A NaN makes its whole row NaN on both.
+ *   Weights holding code 3 (twice the value, which no plane holds) or a lo or hi that is not finite or beyond 2^100
+ * are left to gemm_exact (P2hWeight::planes). */
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+
+constexpr float kXsBig = 5192296858534827628530496329220096.0f;   /* 2^112 */
+
+/* The high halves of two floats as a dword of bf16: lo's in the low half. */
+__device__ __forceinline__ uint32_t hi_halves(float hi, float lo)
+{
+    return perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+}
+__device__ __forceinline__ float cut_bf16(float x) { return __uint_as_float(__float_as_uint(x) & 0xffff0000u); }
+
+/* Eight consecutive values of a row as three bf16 operands, by truncation (every subtraction is exact), in the order
+ * in which decode_planes takes the weights out of a record dword: (1, 3), (0, 2), (5, 7), (4, 6); amax: the largest
+ * magnitude seen. */
+__device__ __forceinline__ void split8(const float (&a)[8], v8bf (&part)[3], float &amax)
+{
+    constexpr int X[4] = {1, 0, 5, 4}, Y[4] = {3, 2, 7, 6};
+    uint32_t p[3][4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const float x = a[X[q]], y = a[Y[q]];
+        p[0][q] = hi_halves(y, x);
+        const float rx = x - cut_bf16(x), ry = y - cut_bf16(y);
+        p[1][q] = hi_halves(ry, rx);
+        p[2][q] = hi_halves(ry - cut_bf16(ry), rx - cut_bf16(rx));
+        asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(amax) : "v"(x), "v"(y));
+    }
+#pragma unroll
+    for (int s = 0; s < 3; s++) part[s] = __builtin_bit_cast(v8bf, make_uint4(p[s][0], p[s][1], p[s][2], p[s][3]));
+}
+
+/* The eight selectors of a record dword as the two planes' operands: ±1/2 is bf16 0x3f00, whose low byte is zero, so
+ * a selector in the odd bytes (and the constant-zero selector 0x0c in the even ones) permutes straight into two
+ * values. Two operations per weight for both planes. */
+__device__ __forceinline__ void decode_planes(uint32_t r, v8bf &lo, v8bf &hi)
+{
+    const uint32_t s[4] = {(r & 0x07000700u) | 0x000c000cu, ((r << 8) & 0x07000700u) | 0x000c000cu,
+                           ((r >> 4) & 0x07000700u) | 0x000c000cu, ((r << 4) & 0x07000700u) | 0x000c000cu};
+    uint32_t wl[4], wh[4];
+#pragma unroll
+    for (int d = 0; d < 4; d++) {
+        wl[d] = perm(0u, 0x003f00bfu, s[d]);
+        wh[d] = perm(0x003f00bfu, 0u, s[d]);
+    }
+    lo = __builtin_bit_cast(v8bf, make_uint4(wl[0], wl[1], wl[2], wl[3]));
+    hi = __builtin_bit_cast(v8bf, make_uint4(wh[0], wh[1], wh[2], wh[3]));
+}
+
+/* Outputs (m, n .. n + 3) as one chain of fmaf over k with the weights expanded as the reference expands them. */
+__device__ __forceinline__ v4f xs_big_row(const ExactArgs &g, int m, int n)
+{
+    v4f sum = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int k = 0; k < g.K; k++) {
+        const float a = g.A[(size_t)m * g.lda + k];
+        int shift;
+        const uint8_t *rb = g.rec + rec_quad_offset(g.units, k & ~3, n, shift) + (k & 3);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int sel = (rb[16 * e] >> shift) & 7;
+            const float lo = g.lo[n + e];
+            sum[e] = __builtin_fmaf(a, (float)((sel & 3) - 1) * __builtin_fmaf((float)(sel >> 2), g.hi[n + e] - lo, lo),
+                                    sum[e]);
+        }
+    }
+    return sum;
+}
+
+/* The exact-mode five-value GEMM (sgemm_fvb_exact, blas.c:929-987): C = beta·C + alpha·A·W with exact products on the
+ * bf16 matrix cores (above), for up to a few hundred rows. The sum runs in a different order from the reference's
+ * per-output fmaf chain (which gemm_exact keeps bit for bit), so outputs agree to fp32 rounding.
  * A workgroup of four waves owns a BM × BN tile and splits K among its waves, as gemm_fvs does: each wave streams its
- * units' weight records (the 4-bit selectors of fv_repack4) and fp32 rows, expands the weights in registers and
- * multiplies; lane l of the step t MFMA takes k = 16·(l / 16) + t of a 64-row step, which is the record's own order.
- * The four partial tiles meet in LDS and are added in wave order.
- * The fp32 rows reach the lanes in one of two ways, with the same MFMAs in the same order (the same bits):
+ * units' weight records (the 4-bit selectors of fv_repack4) and fp32 rows and splits and decodes both in registers;
+ * lane l takes k = 16·(l / 16) .. + 15 of a 64-row step, which is the record's own order. The four partial tiles meet
+ * in LDS and are added in wave order.
+ * The fp32 rows reach the lanes in one of two ways, with the same matrix instructions in the same order (the same
+ * bits). Against the fp32 matrix cores (the same tiles, weights from HBM): M = 375, 1024 → 4096 34.0 → 21.9 µs,
+ * 4096 → 1024 37.8 → 25.4, 1024 → 1024 13.0 → 9.3; M = 125, 1024 → 4096 13.9 → 9.9; M = 38, 4096 → 1024
+ * 11.9 → 10.7. What bounds it now is the split itself (about six VALU operations per value and column tile) and, with
+ * few waves per CU, the loads' latency:
  *   STAGED (K % 128 == 0 and VEC): each wave brings its 64-row K stages of the BM rows into its own LDS slot by
  *     direct loads of whole 256-byte row segments (four rows per instruction, 16-byte chunk c of row r stored at
  *     place c ^ (r % 16), so the operand reads below are free of bank conflicts); no barrier, each wave reads only its
- *     own slot. 43.3 → 31.5 us at M = 375, 1024 → 4096 (16.5 → 12.9 us at 1024 → 1024, 51.9 → 44.1 us at
- *     4096 → 1024): loads straight into the matrix-core layout touch 16 rows × 64 bytes per instruction, and the
- *     lines per instruction, not the bytes, set their pace.
+ *     own slot: loads straight into the matrix-core layout touch 16 rows × 64 bytes per instruction, and the lines
+ *     per instruction, not the bytes, set their pace.
  *   else: loads into registers in the matrix-core layout, units double-buffered.
  * VEC: K % 4 == 0, lda % 4 == 0 and A 16-byte aligned. */
 template <int FM, int FN, bool VEC, bool STAGED = false>
@@ -2923,33 +3020,25 @@ __global__ __launch_bounds__(256, 2) void gemm_xf(ExactArgs g)
     const int nseg = (units + su - 1) / su;
     const int u_begin = min(units, wave * su), u_end = min(units, u_begin + su);
 
-    /* Every weight of column n is one of eight values, w = (code − 1)·fmaf(flag, hi − lo, lo) for the 4-bit
-     * selector code | flag << 2: built once per tile into LDS (rows of 9 floats, so the 16 columns a wave reads
-     * spread over the banks), then one extract and one LDS read per weight. */
-    __shared__ float wtab[BN * 9];
-    for (int c = tid; c < BN * 8; c += NT) {
-        const int col = c >> 3, sel = c & 7, n = min(n0 + col, N - 1);
-        const float lo = g.lo[n], d = g.hi[n] - lo;
-        wtab[col * 9 + sel] = (float)((sel & 3) - 1) * __builtin_fmaf((float)(sel >> 2), d, lo);
-    }
-    int tcol[FN];
+    __shared__ int big[BM];   /* 1: a row that xs_big_row sums */
+    for (int c = tid; c < BM; c += NT) big[c] = 0;
     const uint8_t *b_base[FN];
 #pragma unroll
-    for (int i = 0; i < FN; i++) {
-        const int n = min(n0 + 16 * i + (lane & 15), N - 1);
-        tcol[i] = (16 * i + (lane & 15)) * 9;
-        b_base[i] = g.rec + (size_t)(n >> 4) * units * 1024 + lane * 16;
-    }
+    for (int i = 0; i < FN; i++)
+        b_base[i] = g.rec + (size_t)min((n0 >> 4) + i, N / 16 - 1) * units * 1024 + lane * 16;
     __syncthreads();
     const float *a_row[FM];
 #pragma unroll
     for (int j = 0; j < FM; j++) a_row[j] = g.A + (size_t)min(m0 + 16 * j + (lane & 15), M - 1) * g.lda;
 
-    v4f acc[FN][FM];
+    v4f accL[FN][FM], accH[FN][FM];
+    float amax[FM];
 #pragma unroll
-    for (int i = 0; i < FN; i++)
+    for (int j = 0; j < FM; j++) {
+        amax[j] = 0.0f;
 #pragma unroll
-        for (int j = 0; j < FM; j++) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int i = 0; i < FN; i++) accL[i][j] = accH[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    }
 
     auto load_x = [&](int j, int k0, float x[16]) __attribute__((always_inline)) {
         if (VEC) {
@@ -2961,20 +3050,30 @@ __global__ __launch_bounds__(256, 2) void gemm_xf(ExactArgs g)
     };
 
     uint32_t r[2][FN][4];
-    /* one 64-row step s of a unit whose records are r[rb]: 16 MFMA steps, each weight expanded once for the FM rows */
+    /* one 64-row step s of a unit whose records are r[rb]: k = 16 grp .. + 7, then + 8 .. + 15; smallest part first */
     auto mma_step = [&](int rb, int s, const float (&x)[FM][16]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int t = 0; t < 16; t++) {
-            const int d = t >> 2, b = t & 3;
-            float w[FN];
+        for (int h = 0; h < 2; h++) {
+            v8bf a[FM][3];
 #pragma unroll
-            for (int i = 0; i < FN; i++)
-                w[i] = wtab[tcol[i] + ((r[rb][i][2 * s + (d >> 1)] >> (8 * b + 4 * (d & 1))) & 7u)];
+            for (int j = 0; j < FM; j++) {
+                float x8[8];
 #pragma unroll
-            for (int j = 0; j < FM; j++)
+                for (int e = 0; e < 8; e++) x8[e] = x[j][8 * h + e];
+                split8(x8, a[j], amax[j]);
+            }
 #pragma unroll
-                for (int i = 0; i < FN; i++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i], x[j][t], acc[i][j], 0, 0, 0);
+            for (int i = 0; i < FN; i++) {
+                v8bf wl, wh;
+                decode_planes(r[rb][i][2 * s + h], wl, wh);
+#pragma unroll
+                for (int p = 2; p >= 0; p--)
+#pragma unroll
+                    for (int j = 0; j < FM; j++) {
+                        accL[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wl, a[j][p], accL[i][j], 0, 0, 0);
+                        accH[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wh, a[j][p], accH[i][j], 0, 0, 0);
+                    }
+            }
         }
     };
     auto load_records = [&](int rb, int u) __attribute__((always_inline)) {
@@ -3015,10 +3114,7 @@ __global__ __launch_bounds__(256, 2) void gemm_xf(ExactArgs g)
             }
             mma_step(0, st & 1, x);
         };
-        /* one slot per wave, every load waited before its stage is multiplied: the other waves of the CU (up to four
-         * per SIMD: 34 KB of LDS and at most 128 VGPRs per wave) cover each wave's wait. Two slots per wave with the
-         * next stage in flight measured 5-14 % slower (the doubled LDS halves the workgroups per CU), and eight
-         * waves splitting K no faster. */
+        /* one slot per wave, every load waited before its stage is multiplied: the other waves of the CU cover it */
         for (int st = 0; st < n_st; st += 2) {
             issue(st);        /* step 0 of the unit and its records */
             wait_vm<0>();
@@ -3051,13 +3147,29 @@ __global__ __launch_bounds__(256, 2) void gemm_xf(ExactArgs g)
             mma_unit(1);
         }
     }
-    if (wave < nseg) {
+#pragma unroll
+    for (int j = 0; j < FM; j++)
+        if (!(amax[j] < kXsBig)) big[16 * j + (lane & 15)] = 1;
+    if (wave < nseg) {   /* this wave's sums: 2·lo and 2·hi (as the reference expands it) times the planes' */
         float *dst = part + wave * TILE;
 #pragma unroll
-        for (int i = 0; i < FN; i++)
+        for (int i = 0; i < FN; i++) {
+            const int n = min(n0 + 16 * i + 4 * grp, N - 4);
+            float lo[4], hi[4];
 #pragma unroll
-            for (int j = 0; j < FM; j++)
-                *reinterpret_cast<v4f *>(dst + (16 * j + (lane & 15)) * PITCH + 16 * i + 4 * grp) = acc[i][j];
+            for (int e = 0; e < 4; e++) {
+                lo[e] = g.lo[n + e];
+                hi[e] = 2.0f * __builtin_fmaf(1.0f, g.hi[n + e] - lo[e], lo[e]);
+                lo[e] *= 2.0f;
+            }
+#pragma unroll
+            for (int j = 0; j < FM; j++) {
+                v4f f;
+#pragma unroll
+                for (int e = 0; e < 4; e++) f[e] = __builtin_fmaf(lo[e], accL[i][j][e], hi[e] * accH[i][j][e]);
+                *reinterpret_cast<v4f *>(dst + (16 * j + (lane & 15)) * PITCH + 16 * i + 4 * grp) = f;
+            }
+        }
     }
     __syncthreads();
 
@@ -3069,6 +3181,7 @@ __global__ __launch_bounds__(256, 2) void gemm_xf(ExactArgs g)
         if (m >= M) break;
         v4f sum = *reinterpret_cast<const v4f *>(part + row * PITCH + 4 * cq);
         for (int sg = 1; sg < nseg; sg++) sum += *reinterpret_cast<const v4f *>(part + sg * TILE + row * PITCH + 4 * cq);
+        if (big[row]) sum = xs_big_row(g, m, n);
         float *cp = g.C + (size_t)m * g.ldc + n;
         if (n + 3 < N && (reinterpret_cast<uintptr_t>(cp) & 15) == 0) {   /* one 16-byte store */
             v4f c0 = v4f{0.0f, 0.0f, 0.0f, 0.0f};

@@ -637,6 +637,46 @@ def test_exact_staged_rows_match_register_path(monkeypatch, M, K, N, lda, ldc, t
     _assert_exact(got[rows, :N], ref)
 
 
+@pytest.mark.parametrize("M,K,N", [(2050, 100, 2064), (1090, 1156, 4096), (4099, 64, 1040), (2049, 192, 2048),
+                                    (6000, 640, 704), (37, 200, 80), (130, 1024, 208), (9, 100, 32)])
+def test_exact_split_rows(monkeypatch, M, K, N):
+    """The exact route's split products (gemm_xs' 64 x 128 tiles with cut rows, columns and K steps, and gemm_xf)
+    against the fmaf chain, per row: within (K + 8) fp32 roundings of the sum of magnitudes. Rows with infinities, NaN
+    and values near the largest float give the chain's own infinities, NaN and values."""
+    print(f"exact split M={M} K={K} N={N}", flush=True)
+    signs, flags, lo, hi = _weight(K, N, 960 + N)
+    w = P.FvWeight(signs, flags, lo, hi, K, N)
+    A = P.gen_activations(SEED, 961 + M, M, K)
+    A[1, 5], A[2, 7], A[3, K - 1], A[4, 0] = np.inf, np.nan, -np.inf, 3.0e38
+    A[5] *= np.float32(1e34)
+    A[6] *= np.float32(1e-25)
+    A[7, 3], A[7, 4] = np.inf, -np.inf
+    got = P.fvb_gemm("exact", A, w)
+    ref = _chain(monkeypatch, lambda: P.fvb_gemm("exact", A, w))
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    fin = np.isfinite(ref)
+    assert np.array_equal(got[~fin & ~np.isnan(ref)], ref[~fin & ~np.isnan(ref)])
+    top = np.maximum(np.abs(lo), np.abs(hi)).astype(np.float64)
+    mag = np.where(np.isfinite(A), np.abs(A.astype(np.float64)), 0.0).sum(1)[:, None] * top[None, :]
+    err = np.abs(np.where(fin, got, 0).astype(np.float64) - np.where(fin, ref, 0))
+    assert (err <= (K + 8) * 2.0 ** -24 * mag + 1e-45).all()
+
+
+def test_exact_code3_and_infinite_columns(monkeypatch):
+    """Weights the plane kernels cannot hold (a code 3, an infinite hi) take the fmaf chain: its bits."""
+    K, N, M = 128, 64, 40
+    signs, flags, lo, hi = (a.copy() for a in _weight(K, N, 970))
+    A = P.gen_activations(SEED, 971, M, K)
+    s3 = signs.copy()
+    s3[5, 2] |= 3
+    h_inf = hi.copy()
+    h_inf[9] = np.inf
+    for sg, h in ((s3, hi), (signs, h_inf)):
+        w = P.FvWeight(sg, flags, lo, h, K, N)
+        got = P.fvb_gemm("exact", A, w)
+        assert _bits_equal(got, _chain(monkeypatch, lambda: P.fvb_gemm("exact", A, w)))
+
+
 # ── every tile configuration and K split (the planner's choices forced through its tuning variables) ─────────────
 
 _TILE_CASES = {}
