@@ -178,8 +178,8 @@ int p2h_fvb_gemm_q8a_next(int mode, int M, int N, int K, float alpha, const sign
                           size_t workspace_bytes, const P2hWeight *next, void *stream);
 /* C [M][N] = SiLU(alpha·A·W) (beta 0, ldc = N, N % 8 == 0): the feed-forward's up-projection followed by the SiLU
  * that p2_swish_quant_rows applies before quantising (tensor_ops.c:491-511, encoder.c:345-346), as the AVX2 body's
- * polynomial per element, the same bits as p2h_fvb_gemm_q8a then p2h_silu. The small-M tiles and the int8w large-M
- * tiles apply it as they store C; the others run a second kernel. */
+ * polynomial per element, the same bits as p2h_fvb_gemm_q8a then p2h_silu. The small-M tiles and the large-M tiles
+ * with records in registers apply it as they store C; the others run a second kernel. */
 int p2h_fvb_gemm_q8a_silu(int mode, int M, int N, int K, float alpha, const signed char *dQ, int ldq,
                           const float *dScales, const P2hWeight *w, float *dC, void *workspace,
                           size_t workspace_bytes, void *stream);

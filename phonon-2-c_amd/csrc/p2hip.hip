@@ -138,7 +138,7 @@ struct Switches {
     std::atomic<int> tile{kUnset};          /* P2H_TILE: force a five-value tile */
     std::atomic<int> split_rows{0};         /* P2H_SPLIT_ROWS: force a K split (-1: never) */
     std::atomic<int> xf_staged{1};          /* P2H_XF_STAGED: 0 loads the exact route's rows into registers */
-    std::atomic<int> xf_tile{0};            /* P2H_XF_TILE: force the exact route's tile: 32 or 64 columns of 32 rows,
+    std::atomic<int> xf_tile{0};            /* P2H_XF_TILE: force gemm_xf and its tile: 32 or 64 columns of 32 rows,
                                                or 1616, 1632, 1664 for 16 rows of 16, 32, 64 columns */
     std::atomic<int> exact_chain{0};        /* P2H_EXACT_CHAIN: the exact route's per-output fmaf chain */
     std::atomic<int> sgemm_any{0};          /* P2H_SGEMM_ANY: the fp32 GEMM's element loads */
@@ -1174,8 +1174,8 @@ Plan make_plan(int mode, int M, int N, int K, bool can_split)
          *    segments' loads are all in flight, where those tiles fill between half and all of the CUs;
          *  - K <= 1024: 48 × 64 for wide outputs at a few hundred rows (N >= 3072, M >= 256; 32 × 32 wins up to
          *    N = 2048), else 32 × 32.
-         * Beyond a thousand rows: the two-workgroups-per-CU tiles on 4-bit records (int8w) or 128 × 128 (the
-         * two-plane mode needs twice the accumulators). */
+         * Beyond a thousand rows: the two-workgroups-per-CU tiles on 4-bit records, or 128 × 128 (the two-plane mode
+         * beyond one fold block). */
         const int cus_ = g_cus > 0 ? g_cus : 256;
         auto tiles_of = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
         const long long sd_tiles = tiles_of(SmD::BM, SmD::BN);
@@ -1201,9 +1201,16 @@ Plan make_plan(int mode, int M, int N, int K, bool can_split)
         const long long w6_tiles = (long long)((M + 95) / 96) * ((N + 255) / 256);
         cfg = mode == P2H_INT8W ? (K > p2k::kFoldRows || w6_tiles <= cus_ ? FV_WK : FV_W6) : FV_L;
     }
+    /* The two-plane mode's twice the accumulators fit the 96 × 128 tile with records in registers while no running
+     * outputs are held beside them (one fold block): two workgroups per CU instead of one of the 128 × 128 ring tiles
+     * (M = 1501, 1024 → 3072: the call with its quantiser 29.0 → 16.2 µs; its 288 tiles ran as one full round and an
+     * eighth of another). */
+    const bool plane_rb = mode == P2H_INT8 && M > 1024 && K <= p2k::kFoldRows && switch_of(g_sw.tile) == kUnset &&
+                          switch_of(g_sw.split_rows) <= 0 && switch_of(g_sw.records_in_regs) != 0;
+    if (plane_rb) cfg = FV_WK;
     if (switch_of(g_sw.tile) != kUnset) cfg = switch_of(g_sw.tile);
     if (cfg < 0 || cfg >= FV_COUNT) cfg = FV_S;
-    if (mode == P2H_INT8 && (cfg == FV_X || cfg == FV_W6 || cfg == FV_WK)) cfg = FV_L;
+    if (mode == P2H_INT8 && !plane_rb && (cfg == FV_X || cfg == FV_W6 || cfg == FV_WK)) cfg = FV_L;
     if (mode == P2H_INT8 && int8w_only(cfg)) cfg = FV_SS;
     if (is_small(cfg) && !small_ok(K)) cfg = FV_T;
     /* these never split K across workgroups: the fold stays in the kernel */
@@ -1267,9 +1274,9 @@ p2k::GemmArgs gemm_args(int M, int N, int K, float alpha, float beta, const sign
 }
 
 /* the plan runs on gemm_fv_rb */
-bool records_in_regs(const Plan &p, int mode)
+bool records_in_regs(const Plan &p)
 {
-    return (p.cfg == FV_W6 || p.cfg == FV_WK) && mode != P2H_INT8 && switch_of(g_sw.records_in_regs) != 0;
+    return (p.cfg == FV_W6 || p.cfg == FV_WK) && switch_of(g_sw.records_in_regs) != 0;
 }
 
 /* the large-M tiles: unsplit, two workgroups per CU, 4-bit records (in registers, or through the LDS ring with the
@@ -1333,7 +1340,14 @@ void launch_fv_cfg(const p2k::GemmArgs &g, const Plan &p, hipStream_t s)
     case FV_S8: launch_fv<FvS8, MODE>(g, p, s); break;
     case FV_T6: launch_fv<FvT6, MODE>(g, p, s); break;
     case FV_W6: if (MODE == p2k::MODE_INT8W) { launch_fv_large<FvW6>(g, p, s); break; } /* fall through */
-    case FV_WK: if (MODE == p2k::MODE_INT8W) { launch_fv_large<FvWK>(g, p, s); break; } /* fall through */
+    case FV_WK:
+        if (MODE == p2k::MODE_INT8W) { launch_fv_large<FvWK>(g, p, s); break; }
+        {   /* the two-plane mode: one fold block (make_plan) */
+            const dim3 grid((unsigned)((size_t)p.tiles_m * p.tiles_n)), block(FvWK::NT);
+            if (g.act) hipLaunchKernelGGL((p2k::gemm_fv_rb<FvWK, false, true, p2k::MODE_INT8>), grid, block, 0, s, g);
+            else hipLaunchKernelGGL((p2k::gemm_fv_rb<FvWK, false, false, p2k::MODE_INT8>), grid, block, 0, s, g);
+        }
+        break;
     case FV_X: if (MODE == p2k::MODE_INT8W) { launch_fv<FvX, p2k::MODE_INT8W>(g, p, s); break; } /* fall through */
     default: launch_fv<FvL, MODE>(g, p, s); break;
     }
@@ -1367,7 +1381,7 @@ const char *p2h_fvb_plan(int mode, int M, int N, int K, int with_workspace)
         snprintf(buf, sizeof buf, "tile %dx%d, %d split%s of %d rows%s%s", kFvBM[p.cfg], kFvBN[p.cfg], p.splits,
                  p.splits > 1 ? "s" : "", p.split_rows,
                  p.splits > 1 ? " + fold" : (K > p2k::kFoldRows ? ", folds in registers" : ""),
-                 records_in_regs(p, mode) ? ", weight records in registers" : "");
+                 records_in_regs(p) ? ", weight records in registers" : "");
     return buf;
 }
 
@@ -1438,7 +1452,7 @@ static int fvb_gemm_q8a(int mode, int M, int N, int K, float alpha, const signed
         g.warm = next->rec4;
         g.warm_lines = (int)std::min<size_t>((bytes + 127) / 128, 0x7fffffff);
     }
-    const bool silu_here = silu && (is_small(p.cfg) || records_in_regs(p, mode));
+    const bool silu_here = silu && (is_small(p.cfg) || records_in_regs(p));
     g.act = silu_here ? 1 : 0;
     if (mode == P2H_INT8W) {
         g.c1 = w->hi; g.c1_hi = 1;

@@ -2173,18 +2173,21 @@ __device__ __forceinline__ void fv_tile(const GemmArgs &g)
  *  decodes step 0 of stage t + 1 among stage t's step-1 MFMAs: a stage starts on MFMAs as soon as its first
  *  activation operands are read from LDS. Only the activation operands go through the LDS ring (direct loads, one
  *  barrier per stage). Against the records in LDS: M = 1500 11.3 against 12.4 µs, M = 4099 24.8 against 27.1,
- *  M = 6000 32.5 against 33.7 (1024 → 4096). Two workgroups per CU; the output is folded and staged as in
+ *  M = 6000 32.5 against 33.7 (1024 → 4096). The two-plane mode
+ *  (K <= 1024) runs the 96 × 128 tile with two decoded operands and two sets of sums: M = 1501, 1024 → 3072 24 → 11 µs
+ *  against the 128 × 128 tiles of fv_tile. Two workgroups per CU; the output is folded and staged as in
  *  fv_tile (per 1024-row block, in order; C staged through LDS as whole row segments at device scope). */
-template <class G, bool MULTI, bool ACT>
+template <class G, int MODE, bool MULTI, bool ACT>
 __device__ __forceinline__ void fv_tile_rb(const GemmArgs &g)
 {
+    constexpr bool TWO = MODE == MODE_INT8;
     constexpr int FM = G::FM, FN = G::FN, NW = G::NW, D = G::D, A_STAGE = G::A_STAGE, A_DMA = G::A_DMA;
     constexpr int UNITS_PER_FOLD = kFoldRows / 128;
     constexpr int SROW = G::BN + 4;                    /* staged C rows, padded */
     constexpr int CJ = FM < 3 ? FM : 3;                /* row groups per staging chunk */
     constexpr int RING = D * A_STAGE, STG = 16 * CJ * SROW * 4;
     __shared__ __attribute__((aligned(16))) int8_t ring[RING > STG ? RING : STG];
-    __shared__ __attribute__((aligned(16))) float f_c1[G::BN], f_as[G::BM];
+    __shared__ __attribute__((aligned(16))) float f_c1[G::BN], f_c2[TWO ? G::BN : 4], f_as[G::BM];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int tile_n, tile_m, split;
@@ -2209,7 +2212,7 @@ __device__ __forceinline__ void fv_tile_rb(const GemmArgs &g)
     for (int i = 0; i < FN; i++) {
         const int cg = min((n0 >> 4) + wave * FN + i, g.ng_last);
         b_src[i] = g.rec + (size_t)cg * g.units * 1024 + lane * 16;
-        lo_tab[i] = i8w_lo_table(g.clo[16 * cg + (lane & 15)]);
+        lo_tab[i] = TWO ? 0u : i8w_lo_table(g.clo[16 * cg + (lane & 15)]);
     }
     /* stage t's slot (t % D) filled with stage ts's activation operands (ts = t but past the last stage) */
     auto issue_a = [&](int t, int ts) __attribute__((always_inline)) {
@@ -2219,8 +2222,11 @@ __device__ __forceinline__ void fv_tile_rb(const GemmArgs &g)
     };
 
     /* epilogue factors first (so that waiting for them waits for nothing else), then stage 0 */
-    float r_c1 = 0.0f, r_as = 0.0f;
-    if (tid < G::BN) r_c1 = c1_factor(g, min(n0 + tid, N - 1));
+    float r_c1 = 0.0f, r_c2 = 0.0f, r_as = 0.0f;
+    if (tid < G::BN) {
+        r_c1 = c1_factor(g, min(n0 + tid, N - 1));
+        if (TWO) r_c2 = c2_factor(g, min(n0 + tid, N - 1));
+    }
     if (tid < G::BM) r_as = g.a_scales[min(m0 + tid, M - 1)];
     v4u rb0[FN], rb1[FN];
 #pragma unroll
@@ -2228,24 +2234,33 @@ __device__ __forceinline__ void fv_tile_rb(const GemmArgs &g)
 #pragma unroll
     for (int t = 0; t < D - 1; t++) issue_a(t, min(t, nst - 1));
     if (tid < G::BN) f_c1[tid] = r_c1;
+    if (TWO && tid < G::BN) f_c2[tid] = r_c2;
     if (tid < G::BM) f_as[tid] = r_as * g.alpha;
 
-    auto decode = [&](auto step_tag, const v4u(&rb)[FN], v4i(&bw)[FN]) __attribute__((always_inline)) {
+    auto decode = [&](auto step_tag, const v4u(&rb)[FN], v4i(&bw)[FN], v4i(&bt)[TWO ? FN : 1]) __attribute__((always_inline)) {
         constexpr int S = decltype(step_tag)::value;
 #pragma unroll
         for (int i = 0; i < FN; i++)
 #pragma unroll
             for (int d = 0; d < 4; d++) {
                 const uint32_t sel = (rb[i][2 * S + (d >> 1)] >> (4 * (d & 1))) & 0x07070707u;
-                bw[i][d] = (int)perm(kI8wHiTable, lo_tab[i], sel);
+                if (TWO) {
+                    bw[i][d] = (int)perm(kPlaneS, kPlaneS, sel);
+                    bt[TWO ? i : 0][d] = (int)perm(kPlaneS, 0u, sel);
+                } else {
+                    bw[i][d] = (int)perm(kI8wHiTable, lo_tab[i], sel);
+                }
             }
     };
 
-    v4i acc[FN][FM];
+    v4i acc[FN][FM], accT[TWO ? FN : 1][TWO ? FM : 1];
 #pragma unroll
     for (int i = 0; i < FN; i++)
 #pragma unroll
-        for (int j = 0; j < FM; j++) acc[i][j] = v4i{0, 0, 0, 0};
+        for (int j = 0; j < FM; j++) {
+            acc[i][j] = v4i{0, 0, 0, 0};
+            if (TWO) accT[TWO ? i : 0][TWO ? j : 0] = v4i{0, 0, 0, 0};
+        }
     const int n_lane = n0 + wave * 16 * FN + 4 * (lane >> 4);   /* outputs (m_lane + 16 j, n_lane + 16 i + r) */
     const int m_lane = m0 + (lane & 15);
     const bool beta_zero = g.beta == 0.0f;
@@ -2258,6 +2273,8 @@ __device__ __forceinline__ void fv_tile_rb(const GemmArgs &g)
         for (int i = 0; i < FN; i++) {
             const int nl = wave * 16 * FN + 16 * i + 4 * (lane >> 4);
             const v4f c1 = *reinterpret_cast<const v4f *>(f_c1 + nl);
+            v4f c2 = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+            if (TWO) c2 = *reinterpret_cast<const v4f *>(f_c2 + nl);
             float cold[CASE == 1 ? FM : 1][4];
             if (CASE == 1) {
 #pragma unroll
@@ -2285,13 +2302,15 @@ __device__ __forceinline__ void fv_tile_rb(const GemmArgs &g)
                 const float as = f_as[16 * j + (lane & 15)];
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
-                    const float f = (float)acc[i][j][r] * c1[r];
+                    float f = (float)acc[i][j][r] * c1[r];
+                    if (TWO) f = __builtin_fmaf((float)accT[TWO ? i : 0][TWO ? j : 0][r], c2[r], f);
                     float &out = run[i][j][r];
                     if (CASE == 0) out = f * as;
                     else if (CASE == 1) out = __builtin_fmaf(f, as, cold[CASE == 1 ? j : 0][r]);
                     else out = __builtin_fmaf(f, as, out);
                 }
                 acc[i][j] = v4i{0, 0, 0, 0};
+                if (TWO) accT[TWO ? i : 0][TWO ? j : 0] = v4i{0, 0, 0, 0};
             }
         }
     };
@@ -2301,11 +2320,11 @@ __device__ __forceinline__ void fv_tile_rb(const GemmArgs &g)
         else fold_case(std::integral_constant<int, 1>{});
     };
 
-    v4i bw0[FN], bw1[FN];
+    v4i bw0[FN], bw1[FN], bt0[TWO ? FN : 1], bt1[TWO ? FN : 1];
     wait_vm<0>();
 #pragma unroll
     for (int i = 0; i < FN; i++) pin16(rb0[i]);
-    decode(std::integral_constant<int, 0>{}, rb0, bw0);
+    decode(std::integral_constant<int, 0>{}, rb0, bw0, bt0);
 
     /* stage t: its records in rc (step 0 already decoded into bw0); the next stage's records into rn */
     /* Loads retire in order: waiting until at most the youngest (D − 2) stages of activation loads are in flight
@@ -2327,15 +2346,19 @@ __device__ __forceinline__ void fv_tile_rb(const GemmArgs &g)
             for (int j = 0; j < FM; j++)
                 av[s2][j] = *reinterpret_cast<const v4i *>(sa + (2 * j + s2) * 1024 + lane * 16);
         /* step 0's MFMAs with step 1's decode among them ... */
-        decode(std::integral_constant<int, 1>{}, rc, bw1);
+        decode(std::integral_constant<int, 1>{}, rc, bw1, bt1);
 #pragma unroll
         for (int j = 0; j < FM; j++)
 #pragma unroll
-            for (int i = 0; i < FN; i++)
+            for (int i = 0; i < FN; i++) {
                 acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bw0[i], av[0][j], acc[i][j], 0, 0, 0);
+                if (TWO)
+                    accT[TWO ? i : 0][TWO ? j : 0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+                        bt0[TWO ? i : 0], av[0][j], accT[TWO ? i : 0][TWO ? j : 0], 0, 0, 0);
+            }
         __builtin_amdgcn_sched_group_barrier(0x100, 2 * FM, 0);
 #pragma unroll
-        for (int x = 0; x < FM * FN; x++) {
+        for (int x = 0; x < FM * FN * (TWO ? 2 : 1); x++) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x002, (FN * 10 + FM * FN - 1) / (FM * FN), 0);
         }
@@ -2344,17 +2367,23 @@ __device__ __forceinline__ void fv_tile_rb(const GemmArgs &g)
         wait_vm<(D - 2) * A_DMA>();
 #pragma unroll
         for (int i = 0; i < FN; i++) pin16(rn[i]);
-        decode(std::integral_constant<int, 0>{}, rn, bw0);
+        decode(std::integral_constant<int, 0>{}, rn, bw0, bt0);
 #pragma unroll
         for (int j = 0; j < FM; j++)
 #pragma unroll
-            for (int i = 0; i < FN; i++)
+            for (int i = 0; i < FN; i++) {
                 acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bw1[i], av[1][j], acc[i][j], 0, 0, 0);
+                if (TWO)
+                    accT[TWO ? i : 0][TWO ? j : 0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+                        bt1[TWO ? i : 0], av[1][j], accT[TWO ? i : 0][TWO ? j : 0], 0, 0, 0);
+            }
 #pragma unroll
-        for (int x = 0; x < FM * FN; x++) {
+        for (int x = 0; x < FM * FN * (TWO ? 2 : 1); x++) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x002, (FN * 10 + FM * FN - 1) / (FM * FN), 0);
         }
+#pragma unroll
+        for (int i = 0; i < (TWO ? FN : 0); i++) asm volatile("" : "+v"(bt0[TWO ? i : 0]));
 #pragma unroll
         for (int i = 0; i < FN; i++) asm volatile("" : "+v"(bw0[i]));   /* made here, not after the loop's branch */
         if (MULTI && t + 1 < nst && (t + 1) % UNITS_PER_FOLD == 0) {
@@ -2412,10 +2441,10 @@ __device__ __forceinline__ void fv_tile_rb(const GemmArgs &g)
  * segments between the staging and the store. As a pass of its own after the GEMM it reads and writes C again:
  * 42 µs at M = 6000, 1024 → 4096, beside the GEMM's 33; here it costs 7 of them (the feed-forward half step at 6000
  * rows 160.3 → 125.1 µs). */
-template <class G, bool MULTI, bool ACT>
+template <class G, bool MULTI, bool ACT, int MODE = MODE_INT8W>
 __global__ __launch_bounds__(G::NT, 2) void gemm_fv_rb(GemmArgs g)
 {
-    fv_tile_rb<G, MULTI, ACT>(g);
+    fv_tile_rb<G, MODE, MULTI, ACT>(g);
 }
 
 template <class G, int MODE, int OUT, bool MULTI, bool SPLIT, int OCC = 1, bool CSHUF = false>
@@ -2905,10 +2934,10 @@ __global__ __launch_bounds__(256) void gemm_exact(ExactArgs g)
  * row's value is cut into three bf16 parts (8 + 8 + 8 significand bits, their sum exactly the value), and the weights
  * into two planes of −1/2, 0, 1/2: the signs where the flag is clear and where it is set. Every product of a part with
  * a plane is exact, the sums are fp32 as on the fp32 matrix cores, and 2·lo and 2·hi scale the two planes' sums at the
- * end: six bf16 matrix instructions of 32 k against eight fp32 ones of 4 k for the same work, at a sixteenth of the
- * time each. No value is rounded on the way in and a 32-k step rounds a sum three times instead of eight, so the
- * outputs are nearer to the 64-bit ones than the fp32 instructions': 1.6e-7 against 2.3e-7 (relative, K = 1024) and
- * 1.7e-7 against 4.5e-7 (K = 4096).
+ * end: six bf16 matrix instructions (16 × 16 × 32) do the work of eight fp32 ones (16 × 16 × 4), each in half the
+ * time. No value is rounded on the way in and a 32-k step rounds a sum three times instead of eight, so the outputs are
+ * nearer to the 64-bit ones than the fp32 instructions' (relative error, K = 1024 and 4096): 1.2e-7 and 2.3e-7 for
+ * gemm_xf, 1.6e-7 and 1.7e-7 for gemm_xs, against 2.3e-7 and 4.5e-7.
  *   Rows holding a value of 2^112 or more (or an infinity, whose parts are not finite) are summed by a scalar chain
  * of fmaf over the expanded weights instead (xs_big_row): the planes' zeros would make NaN of an infinity, and the
  * halves could overflow where the real weights do not. A NaN makes its whole row NaN on both.

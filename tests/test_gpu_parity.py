@@ -378,6 +378,24 @@ def test_q8a_silu_matches_gemm_then_silu(mode, M, K, N):
     assert _bits_equal(got, ref)
 
 
+@pytest.mark.parametrize("M,K,N", [(1025, 1024, 272), (1501, 1024, 3072), (1100, 132, 16), (2000, 900, 144)])
+@pytest.mark.parametrize("beta", [0.0, 1.0, 0.3])
+def test_two_plane_records_in_registers(monkeypatch, M, K, N, beta):
+    """The two-plane mode's 96 x 128 tiles with the records in registers: the bits of the 128 x 128 tiles
+    (P2H_RECORDS_IN_REGISTERS=0), with cut row and column tiles, and of the SiLU after the GEMM."""
+    print(f"two-plane M={M} K={K} N={N} beta={beta} {P.plan('int8', M, N, K)}", flush=True)
+    A = P.gen_activations(SEED, 1970 + M, M, K)
+    q, sc = O.quant_rows(A)
+    w = P.FvWeight(*_weight(K, N, 1980 + N), K, N)
+    C0 = np.random.default_rng(M).standard_normal((M, N)).astype(np.float32)
+    got = P.fvb_gemm_q8a("int8", q, sc, w, alpha=0.7, beta=beta, C0=C0)
+    act = P.fvb_gemm_q8a_silu("int8", q, sc, w, alpha=0.7)
+    monkeypatch.setenv("P2H_RECORDS_IN_REGISTERS", "0")
+    assert "registers" not in P.plan("int8", M, N, K)
+    assert _bits_equal(got, P.fvb_gemm_q8a("int8", q, sc, w, alpha=0.7, beta=beta, C0=C0))
+    assert _bits_equal(act, P.fvb_gemm_q8a_silu("int8", q, sc, w, alpha=0.7))
+
+
 @pytest.mark.parametrize("M,K,N", [(2101, 128, 4112), (1025, 1024, 272), (1030, 1156, 16), (1100, 4096, 144)])
 def test_q8a_silu_large_tiles(M, K, N):
     """The int8w large-M tiles' SiLU (96 x 256 and 96 x 128, one and several fold blocks) with a cut last row tile and
@@ -573,8 +591,8 @@ def test_xcd_grid_same_bits(monkeypatch, M, K, N):
 
 @pytest.mark.parametrize("M,K,N", [(6000, 1024, 4096), (6000, 4096, 1024)])
 def test_exact_full_size_sampled_rows(monkeypatch, M, K, N):
-    """The exact route at the batched long-audio shapes (16 windows stacked, 12k+ workgroups on the fp32 matrix
-    cores): sampled rows (first and last included) within 1e-4 of the oracle's exact route, the fmaf-chain route
+    """The exact route at the batched long-audio shapes (16 windows stacked, split products on the bf16
+    matrix cores): sampled rows (first and last included) within 1e-4 of the oracle's exact route, the fmaf-chain route
     (P2H_EXACT_CHAIN=1) bit-exact on the same rows, and over every row the power-of-two property (rows scaled by 4
     give outputs scaled by exactly 4: every product and partial sum scales exactly)."""
     signs, flags, lo, hi = _weight(K, N, 740 + K + N)
