@@ -14,6 +14,7 @@
 #include <climits>
 #include <atomic>
 #include <mutex>
+#include <vector>
 
 #include "p2hip_kernels.h"
 #include "p2hip_split.h"
@@ -487,24 +488,48 @@ static P2hWeight *weight_new(int K, int N, bool copy_planes)
     return w;
 }
 
+/* Pinned words in which the weight kernels report to the host, one per upload under way (a copy back from device
+ * memory costs an upload 50 µs): as many as have ever been uploading at once, kept until the process ends. */
+static std::mutex g_words_mu;
+static std::vector<uint32_t *> g_words;
+
+static uint32_t *word_take(void)
+{
+    {
+        std::lock_guard<std::mutex> lock(g_words_mu);
+        if (!g_words.empty()) {
+            uint32_t *p = g_words.back();
+            g_words.pop_back();
+            return p;
+        }
+    }
+    void *p = nullptr;
+    return hipHostMalloc(&p, 64, hipHostMallocPortable) == hipSuccess ? (uint32_t *)p : nullptr;
+}
+
 static int weight_tables(P2hWeight *w)
 {
     hipStream_t s = stream_of(nullptr);
-    hipLaunchKernelGGL(p2k::fv_tables, dim3((w->N + 255) / 256), dim3(256), 0, s, w->N, w->lo, w->hi, w->clo);
-    HIPCHK(hipGetLastError());
+    uint32_t *odd = word_take();   /* set by the kernels for what the exact route's plane kernels cannot hold */
+    if (!odd) return fail(P2H_E_NOMEM, "five-value weight: pinned allocation failed");
+    *(volatile uint32_t *)odd = 0;
+    hipLaunchKernelGGL(p2k::fv_tables, dim3((w->N + 255) / 256), dim3(256), 0, s, w->N, w->lo, w->hi, w->clo, odd);
     const size_t recs = (size_t)(w->N / 16) * w->units * 64;
-    uint32_t odd = 0;   /* the word after the records: set by the kernels for what the plane kernels cannot hold */
-    if (recs > 0) {
-        uint32_t *d_odd = (uint32_t *)(w->rec4 + recs * 16);
-        hipLaunchKernelGGL(p2k::fill_u32, dim3(1), dim3(256), 0, s, d_odd, (size_t)1, 0u);
+    if (recs > 0)
         hipLaunchKernelGGL(p2k::fv_repack4, dim3((unsigned)((recs + 255) / 256)), dim3(256), 0, s, w->K, w->N,
-                           w->units, w->signs, w->flags, (uint4 *)w->rec4, d_odd);
-        hipLaunchKernelGGL(p2k::fv_check, dim3((w->N + 255) / 256), dim3(256), 0, s, w->N, w->lo, w->hi, d_odd);
-        HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpyAsync(&odd, d_odd, sizeof odd, hipMemcpyDeviceToHost, s));
+                           w->units, w->signs, w->flags, (uint4 *)w->rec4, odd);
+    const hipError_t launched = hipGetLastError(), done = hipStreamSynchronize(s);
+    w->planes = *(volatile uint32_t *)odd == 0;
+    if (done == hipSuccess) {   /* else a kernel may still write it: left out of the pool */
+        std::lock_guard<std::mutex> lock(g_words_mu);
+        try {
+            g_words.push_back(odd);
+        } catch (...) {   /* no memory for the list: the word goes back instead */
+            (void)hipHostFree(odd);
+        }
     }
-    HIPCHK(hipStreamSynchronize(s));
-    w->planes = odd == 0;
+    HIPCHK(launched);
+    HIPCHK(done);
     return P2H_OK;
 }
 

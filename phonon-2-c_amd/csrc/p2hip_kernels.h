@@ -81,7 +81,10 @@ __device__ __forceinline__ uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel)
 
 /* clo[n] = clamp(lrintf(127·lo/hi), 0, 127), 0 when hi <= 0 (blas.c:1319-1326). The fold's other factors,
  * hi·(1/127) and hi − lo (blas.c:1327-1333), are made from lo and hi where they are used (c1_factor, c2_factor). */
-__global__ void fv_tables(int N, const float *__restrict__ lo, const float *__restrict__ hi, uint8_t *__restrict__ clo)
+/* clo; and *odd = 1 where a column's lo or expanded hi is not finite or is 2^100 or more (the exact route's plane
+ * kernels scale their sums by both, used or not). */
+__global__ void fv_tables(int N, const float *__restrict__ lo, const float *__restrict__ hi, uint8_t *__restrict__ clo,
+                          uint32_t *odd)
 {
     int n = blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= N) return;
@@ -92,6 +95,8 @@ __global__ void fv_tables(int N, const float *__restrict__ lo, const float *__re
         c = r < 0.0f ? 0 : r > 127.0f ? 127 : (int)r;
     }
     clo[n] = (uint8_t)c;
+    const float e = __builtin_fmaf(1.0f, h - l, l), big = 1267650600228229401496703205376.0f;   /* 2^100 */
+    if (!(__builtin_fabsf(l) < big && __builtin_fabsf(e) < big)) *odd = 1u;
 }
 
 /* ── activation quantisation ───────────────────────────────────────────────────────────────────────────────── */
@@ -1782,7 +1787,7 @@ void gemm_i8(GemmArgs g)
  * brings a whole 128-row unit, and an operand dword decodes with one mask (and one shift for odd d) before the
  * table permute. */
 __global__ void fv_repack4(int K, int N, int units, const uint8_t *__restrict__ signs,
-                           const uint8_t *__restrict__ flags, uint4 *__restrict__ rec, uint32_t *__restrict__ odd)
+                           const uint8_t *__restrict__ flags, uint4 *__restrict__ rec, uint32_t *odd)
 {
     const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= (size_t)(N / 16) * units * 64) return;
@@ -1806,16 +1811,6 @@ __global__ void fv_repack4(int K, int N, int units, const uint8_t *__restrict__ 
             }
     if (any3) *odd = 1u;   /* code 3 (twice the value): the exact route's plane kernels cannot hold it */
     rec[idx] = make_uint4(w[0], w[1], w[2], w[3]);
-}
-
-/* *odd = 1 where a column's lo or expanded hi is not finite or is 2^100 or more (the plane kernels scale their sums by
- * both, used or not). */
-__global__ void fv_check(int N, const float *__restrict__ lo, const float *__restrict__ hi, uint32_t *__restrict__ odd)
-{
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= N) return;
-    const float l = lo[n], h = __builtin_fmaf(1.0f, hi[n] - l, l), big = 1267650600228229401496703205376.0f;
-    if (!(__builtin_fabsf(l) < big && __builtin_fabsf(h) < big)) *odd = 1u;
 }
 
 /* The selector nibble (code | flag << 2, fv_repack4's layout) of weight (k, n) lives in record (n / 16, k / 128),
