@@ -489,7 +489,7 @@ static P2hWeight *weight_new(int K, int N, bool copy_planes)
 }
 
 /* Pinned words in which the weight kernels report to the host, one per upload under way (a copy back from device
- * memory costs an upload 50 µs): as many as have ever been uploading at once, kept until the process ends. */
+ * memory cost an upload about 60 µs: 400 -> 467 for a 1024 x 3072 weight): as many as have ever been uploading at once, kept until the process ends. */
 static std::mutex g_words_mu;
 static std::vector<uint32_t *> g_words;
 
