@@ -24,9 +24,20 @@ import p2gemm as P  # noqa: E402
 BLOCK_TID0 = 100
 
 
+def pos_encoding(T):
+    """The sinusoids of positions T − 1 .. −(T − 1), [2T − 1, 1024] (rel_pos_encoding, encoder.c:79-96), in 64 bits."""
+    pos = np.arange(T - 1, -T, -1, dtype=np.float64)[:, None]
+    angle = pos * np.exp(np.arange(0, P.D_MODEL, 2) * (-np.log(10000.0) / P.D_MODEL))
+    pe = np.empty((2 * T - 1, P.D_MODEL))
+    pe[:, 0::2], pe[:, 1::2] = np.sin(angle), np.cos(angle)
+    return pe.astype(np.float32)
+
+
 def block_input(seed, T):
-    """The block's input rows and positional rows: generator activations [T, 1024], rel_pos_encoding (encoder.c:79-96)."""
-    return P.gen_activations(seed, BLOCK_TID0 - 1, T, P.D_MODEL), O.ref_pos_encoding(T)
+    """The block's input rows and positional rows: generator activations [T, 1024] and the reference's own table, or
+    where its library is not built (tests that compare the device block with itself) the one computed here."""
+    pe = O.ref_pos_encoding(T) if O.refblock_available() else pos_encoding(T)
+    return P.gen_activations(seed, BLOCK_TID0 - 1, T, P.D_MODEL), pe
 
 
 RESIDUAL_LINEARS = ("ff1_l2", "out", "pw2", "ff2_l2")   # encoder.c:347, 530, 602, 347: the products added to x
