@@ -2926,21 +2926,23 @@ __global__ __launch_bounds__(256) void gemm_exact(ExactArgs g)
 
 /* ── exact products on the bf16 matrix cores ───────────────────────────────────────────────────────────────────
  * The exact route's products of fp32 rows with five-value weights, w = (code − 1)·v with v = lo or hi by the flag. A
- * row's value is cut into three bf16 parts (8 + 8 + 8 significand bits, their sum exactly the value), and the weights
+ * row's value is cut into three bf16 parts (8 + 8 + 8 significand bits, their sum the value), and the weights
  * into two planes of −1/2, 0, 1/2: the signs where the flag is clear and where it is set. Every product of a part with
  * a plane is exact, the sums are fp32 as on the fp32 matrix cores, and 2·lo and 2·hi scale the two planes' sums at the
  * end: six bf16 matrix instructions (16 × 16 × 32) do the work of eight fp32 ones (16 × 16 × 4), each in half the
  * time. No value is rounded on the way in and a 32-k step rounds a sum three times instead of eight, so the outputs are
  * nearer to the 64-bit ones than the fp32 instructions' (relative error, K = 1024 and 4096): 1.2e-7 and 2.3e-7 for
  * gemm_xf, 1.6e-7 and 1.7e-7 for gemm_xs, against 2.3e-7 and 4.5e-7.
- *   Rows holding a value of 2^112 or more (or an infinity, whose parts are not finite) are summed by a scalar chain
- * of fmaf over the expanded weights instead (xs_big_row): the planes' zeros would make NaN of an infinity, and the
- * halves could overflow where the real weights do not. A NaN makes its whole row NaN on both.
+ *   Outputs that come out infinite or NaN are summed again by a scalar chain of fmaf over the expanded weights
+ * (xs_complete, slow): the planes' zeros make NaN of an infinity's parts, and sums of halves could overflow where those of
+ * the real products do not.
+ *   bf16's smallest step is 2^-133, so of a value below 2^-110 the parts leave bits out: those of the third remainder
+ * below that step. split8 notes that there are any (one operation in twelve of a pair) and xs_complete adds their
+ * products to the row's finished sums, so that small values count in full, alone in a row or beside large ones. The
+ * parts themselves may be denormal: these matrix instructions neither flush them nor the sums.
  *   Weights holding code 3 (twice the value, which no plane holds) or a lo or hi that is not finite or beyond 2^100
  * are left to gemm_exact (P2hWeight::planes). */
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-
-constexpr float kXsBig = 5192296858534827628530496329220096.0f;   /* 2^112 */
 
 /* The high halves of two floats as a dword of bf16: lo's in the low half. */
 __device__ __forceinline__ uint32_t hi_halves(float hi, float lo)
@@ -2950,9 +2952,9 @@ __device__ __forceinline__ uint32_t hi_halves(float hi, float lo)
 __device__ __forceinline__ float cut_bf16(float x) { return __uint_as_float(__float_as_uint(x) & 0xffff0000u); }
 
 /* Eight consecutive values of a row as three bf16 operands, by truncation (every subtraction is exact), in the order
- * in which decode_planes takes the weights out of a record dword: (1, 3), (0, 2), (5, 7), (4, 6); amax: the largest
- * magnitude seen. */
-__device__ __forceinline__ void split8(const float (&a)[8], v8bf (&part)[3], float &amax)
+ * in which decode_planes takes the weights out of a record dword: (1, 3), (0, 2), (5, 7), (4, 6); low: its low half is
+ * not 0 once a value had bits below the parts'. */
+__device__ __forceinline__ void split8(const float (&a)[8], v8bf (&part)[3], uint32_t &low)
 {
     constexpr int X[4] = {1, 0, 5, 4}, Y[4] = {3, 2, 7, 6};
     uint32_t p[3][4];
@@ -2962,8 +2964,10 @@ __device__ __forceinline__ void split8(const float (&a)[8], v8bf (&part)[3], flo
         p[0][q] = hi_halves(y, x);
         const float rx = x - cut_bf16(x), ry = y - cut_bf16(y);
         p[1][q] = hi_halves(ry, rx);
-        p[2][q] = hi_halves(ry - cut_bf16(ry), rx - cut_bf16(rx));
-        asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(amax) : "v"(x), "v"(y));
+        float sx = rx - cut_bf16(rx), sy = ry - cut_bf16(ry);
+        /* low |= sx | sy, tied ahead of the remainders' last use: free to move, it kept all of them in registers */
+        asm("v_or3_b32 %0, %0, %1, %2" : "+v"(low), "+v"(sx), "+v"(sy));
+        p[2][q] = hi_halves(sy, sx);
     }
 #pragma unroll
     for (int s = 0; s < 3; s++) part[s] = __builtin_bit_cast(v8bf, make_uint4(p[s][0], p[s][1], p[s][2], p[s][3]));
@@ -2986,23 +2990,43 @@ __device__ __forceinline__ void decode_planes(uint32_t r, v8bf &lo, v8bf &hi)
     hi = __builtin_bit_cast(v8bf, make_uint4(wh[0], wh[1], wh[2], wh[3]));
 }
 
-/* Outputs (m, n .. n + 3) as one chain of fmaf over k with the weights expanded as the reference expands them. */
-__device__ __forceinline__ v4f xs_big_row(const ExactArgs &g, int m, int n)
+/* What split8's parts leave out of a value (0 from 2^-110 up). */
+__device__ __forceinline__ float left_out(float x)
 {
-    v4f sum = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-    for (int k = 0; k < g.K; k++) {
-        const float a = g.A[(size_t)m * g.lda + k];
-        int shift;
-        const uint8_t *rb = g.rec + rec_quad_offset(g.units, k & ~3, n, shift) + (k & 3);
+    const float r = x - cut_bf16(x), t = r - cut_bf16(r);
+    return t - cut_bf16(t);
+}
+
+/* The finished sums of outputs (m, n .. n + 3) made whole: finite ones take what the parts left out of a row with such
+ * values (low); others are summed again, as one chain of fmaf over k with the weights as the reference expands them. One
+ * loop for both, eight values at a time, since its code lies in every kernel's epilogue. */
+__device__ __forceinline__ v4f xs_complete(const ExactArgs &g, int m, int n, v4f sum, bool low)
+{
+    constexpr float top = 3.402823466e38f;
+    const bool again = !(__builtin_fabsf(sum[0]) <= top && __builtin_fabsf(sum[1]) <= top &&
+                         __builtin_fabsf(sum[2]) <= top && __builtin_fabsf(sum[3]) <= top);
+    if (!again && !low) return sum;
+    const float *row = g.A + (size_t)m * g.lda;
+    v4f rest = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int k0 = 0; k0 < g.K; k0 += 8) {
+        float any = 0.0f;
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int sel = (rb[16 * e] >> shift) & 7;
-            const float lo = g.lo[n + e];
-            sum[e] = __builtin_fmaf(a, (float)((sel & 3) - 1) * __builtin_fmaf((float)(sel >> 2), g.hi[n + e] - lo, lo),
-                                    sum[e]);
+        for (int e = 0; e < 8; e++) any += __builtin_fabsf(left_out(row[min(k0 + e, g.K - 1)]));
+        if (!again && any == 0.0f) continue;
+#pragma unroll 1
+        for (int k = k0; k < min(k0 + 8, g.K); k++) {
+            const float v = again ? row[k] : left_out(row[k]);
+            int shift;
+            const uint8_t *rb = g.rec + rec_quad_offset(g.units, k & ~3, n, shift) + (k & 3);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int sel = (rb[16 * e] >> shift) & 7;
+                const float lo = g.lo[n + e], w = __builtin_fmaf((float)(sel >> 2), g.hi[n + e] - lo, lo);
+                rest[e] = __builtin_fmaf(v, (float)((sel & 3) - 1) * w, rest[e]);
+            }
         }
     }
-    return sum;
+    return again ? rest : sum + rest;
 }
 
 /* The exact-mode five-value GEMM (sgemm_fvb_exact, blas.c:929-987): C = beta·C + alpha·A·W with exact products on the
@@ -3044,8 +3068,8 @@ __global__ __launch_bounds__(256, 2) void gemm_xf(ExactArgs g)
     const int nseg = (units + su - 1) / su;
     const int u_begin = min(units, wave * su), u_end = min(units, u_begin + su);
 
-    __shared__ int big[BM];   /* 1: a row that xs_big_row sums */
-    for (int c = tid; c < BM; c += NT) big[c] = 0;
+    __shared__ int lowbits[BM];   /* 1: a row with values whose parts leave bits out */
+    for (int c = tid; c < BM; c += NT) lowbits[c] = 0;
     const uint8_t *b_base[FN];
 #pragma unroll
     for (int i = 0; i < FN; i++)
@@ -3056,10 +3080,10 @@ __global__ __launch_bounds__(256, 2) void gemm_xf(ExactArgs g)
     for (int j = 0; j < FM; j++) a_row[j] = g.A + (size_t)min(m0 + 16 * j + (lane & 15), M - 1) * g.lda;
 
     v4f accL[FN][FM], accH[FN][FM];
-    float amax[FM];
+    uint32_t low[FM];
 #pragma unroll
     for (int j = 0; j < FM; j++) {
-        amax[j] = 0.0f;
+        low[j] = 0u;
 #pragma unroll
         for (int i = 0; i < FN; i++) accL[i][j] = accH[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     }
@@ -3084,7 +3108,7 @@ __global__ __launch_bounds__(256, 2) void gemm_xf(ExactArgs g)
                 float x8[8];
 #pragma unroll
                 for (int e = 0; e < 8; e++) x8[e] = x[j][8 * h + e];
-                split8(x8, a[j], amax[j]);
+                split8(x8, a[j], low[j]);
             }
 #pragma unroll
             for (int i = 0; i < FN; i++) {
@@ -3125,8 +3149,8 @@ __global__ __launch_bounds__(256, 2) void gemm_xf(ExactArgs g)
             for (int q = 0; q < NQ; q++) dma_16(a_src[q] + 128 * u + 64 * (st & 1), slot + q * 1024);
             if ((st & 1) == 0) load_records(0, u);
         };
-        auto compute = [&](int st) __attribute__((always_inline)) {
-            float x[FM][16];
+        float x[FM][16];
+        auto read = [&]() __attribute__((always_inline)) {
 #pragma unroll
             for (int j = 0; j < FM; j++) {
                 const int8_t *row = slot + (16 * j + (lane & 15)) * 256;
@@ -3136,16 +3160,20 @@ __global__ __launch_bounds__(256, 2) void gemm_xf(ExactArgs g)
                     x[j][4 * q4] = v.x; x[j][4 * q4 + 1] = v.y; x[j][4 * q4 + 2] = v.z; x[j][4 * q4 + 3] = v.w;
                 }
             }
-            mma_step(0, st & 1, x);
         };
-        /* one slot per wave, every load waited before its stage is multiplied: the other waves of the CU cover it */
+        /* one slot per wave: step 1 loads while step 0 is multiplied (the barriers keep it so), the wait for step 0
+         * is covered by the other waves of the CU */
         for (int st = 0; st < n_st; st += 2) {
             issue(st);        /* step 0 of the unit and its records */
             wait_vm<0>();
-            compute(st);
+            read();
             issue(st + 1);    /* step 1 */
+            __builtin_amdgcn_sched_barrier(0);
+            mma_step(0, 0, x);
+            __builtin_amdgcn_sched_barrier(0);
             wait_vm<0>();
-            compute(st + 1);
+            read();
+            mma_step(0, 1, x);
         }
         __syncthreads();   /* every wave is done with its slots: the partial tiles reuse the area */
     } else {
@@ -3173,7 +3201,7 @@ __global__ __launch_bounds__(256, 2) void gemm_xf(ExactArgs g)
     }
 #pragma unroll
     for (int j = 0; j < FM; j++)
-        if (!(amax[j] < kXsBig)) big[16 * j + (lane & 15)] = 1;
+        if (low[j] & 0xffffu) lowbits[16 * j + (lane & 15)] = 1;
     if (wave < nseg) {   /* this wave's sums: 2·lo and 2·hi (as the reference expands it) times the planes' */
         float *dst = part + wave * TILE;
 #pragma unroll
@@ -3205,7 +3233,7 @@ __global__ __launch_bounds__(256, 2) void gemm_xf(ExactArgs g)
         if (m >= M) break;
         v4f sum = *reinterpret_cast<const v4f *>(part + row * PITCH + 4 * cq);
         for (int sg = 1; sg < nseg; sg++) sum += *reinterpret_cast<const v4f *>(part + sg * TILE + row * PITCH + 4 * cq);
-        if (big[row]) sum = xs_big_row(g, m, n);
+        sum = xs_complete(g, m, n, sum, lowbits[row] != 0);
         float *cp = g.C + (size_t)m * g.ldc + n;
         if (n + 3 < N && (reinterpret_cast<uintptr_t>(cp) & 15) == 0) {   /* one 16-byte store */
             v4f c0 = v4f{0.0f, 0.0f, 0.0f, 0.0f};

@@ -33,7 +33,7 @@ __global__ __launch_bounds__(G::NT, 2) void gemm_xs(ExactArgs g)
     constexpr int FM = G::FM, FN = G::FN, BM = G::BM, BN = G::BN, NT = G::NT, NO = G::NO, STEP = G::STEP;
     __shared__ __attribute__((aligned(16))) int8_t ring[2 * STEP];
     __shared__ __attribute__((aligned(16))) float f_lo[BN], f_hi[BN];
-    __shared__ int big[BM];
+    __shared__ int lowbits[BM];   /* 1: a row with values whose parts leave bits out */
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, grp = lane >> 4, x = lane & 15;
     const int wm = wave / G::WN, wn = wave % G::WN;
@@ -54,21 +54,21 @@ __global__ __launch_bounds__(G::NT, 2) void gemm_xs(ExactArgs g)
         f_lo[c] = 2.0f * lo;
         f_hi[c] = 2.0f * hi;
     }
-    for (int c = tid; c < BM; c += NT) big[c] = 0;
+    for (int c = tid; c < BM; c += NT) lowbits[c] = 0;
 
     /* octet q of this thread: row orow, k = 64 t + 8 o; its place in a part's 1 KB block of (16 rows, half h):
      * operand lane (o / 2, row % 16), the row turned by 4 (o / 2) + 2 h so that the eight octets of a row land on
      * eight different 16-byte columns of the banks */
     const float *asrc[NO];
     int adst[NO];
-    float amax[NO];
+    uint32_t low[NO];
     const int o = tid & 7;
 #pragma unroll
     for (int q = 0; q < NO; q++) {
         const int row = min((tid >> 3) + q * (NT / 8), BM - 1);
         asrc[q] = g.A + (size_t)min(m0 + row, M - 1) * g.lda + 8 * o;
         adst[q] = ((row >> 4) * 2 + (o & 1)) * 3072 + ((o >> 1) * 16 + ((row & 15) ^ (2 * o))) * 16;
-        amax[q] = 0.0f;
+        low[q] = 0u;
     }
     auto has = [&](int q) __attribute__((always_inline)) { return (q + 1) * NT <= BM * 8 || tid + q * NT < BM * 8; };
     const uint8_t *b_src[FN];
@@ -101,7 +101,7 @@ __global__ __launch_bounds__(G::NT, 2) void gemm_xs(ExactArgs g)
                 for (int e = 0; e < 8; e++) av[q][e] = k + (e & 4) < K ? av[q][e] : 0.0f;
             }
             v8bf p[3];
-            split8(av[q], p, amax[q]);
+            split8(av[q], p, low[q]);
 #pragma unroll
             for (int s = 0; s < 3; s++)
                 *reinterpret_cast<v8bf *>(ring + buf * STEP + adst[q] + 1024 * s) = p[s];
@@ -185,7 +185,7 @@ __global__ __launch_bounds__(G::NT, 2) void gemm_xs(ExactArgs g)
     fold();
 #pragma unroll
     for (int q = 0; q < NO; q++)
-        if (has(q) && !(amax[q] < kXsBig)) big[(tid >> 3) + q * (NT / 8)] = 1;
+        if (has(q) && (low[q] & 0xffffu)) lowbits[(tid >> 3) + q * (NT / 8)] = 1;
     lds_barrier();   /* every wave is done with the ring: the outputs are staged in it */
     float *stg = reinterpret_cast<float *>(ring);
 #pragma unroll
@@ -203,7 +203,7 @@ __global__ __launch_bounds__(G::NT, 2) void gemm_xs(ExactArgs g)
         const int m = m0 + row;
         if (m >= M) break;
         v4f sum = *reinterpret_cast<const v4f *>(stg + row * G::PITCH + 4 * cq);
-        if (big[row]) sum = xs_big_row(g, m, n);
+        sum = xs_complete(g, m, n, sum, lowbits[row] != 0);
         float *cp = g.C + (size_t)m * g.ldc + n;
         v4f c0 = v4f{0.0f, 0.0f, 0.0f, 0.0f};
         if (g.beta != 0.0f) {

@@ -680,6 +680,43 @@ def test_exact_split_rows(monkeypatch, M, K, N):
     assert (err <= (K + 8) * 2.0 ** -24 * mag + 1e-45).all()
 
 
+def _expand64(signs, flags, lo, hi, N):
+    """The weights [K][N] as the reference expands them to fp32 (blas.c:875-897), held in 64 bits."""
+    code = ((signs[:, :, None] >> (2 * np.arange(4, dtype=np.uint8))) & 3).reshape(len(signs), N)
+    flag = np.unpackbits(flags, axis=1, bitorder="little")[:, :N]
+    return (code - 1.0) * np.where(flag != 0, lo + (hi - lo), lo).astype(np.float64)
+
+
+@pytest.mark.parametrize("M,K,N", [(40, 1024, 64), (37, 100, 80), (21, 1001, 48), (2050, 128, 2064), (2050, 100, 2064)])
+@pytest.mark.parametrize("grow", [1.0, 2.0 ** 70])
+def test_exact_small_values(M, K, N, grow):
+    """Values down to the smallest float count in full on the exact route, whole rows of them and beside ordinary
+    values, and a row near the largest float: every output within K + 8 fp32 roundings of its own products' magnitudes
+    (and of fp32's smallest step), with the format's lo and hi and with ones that bring such rows back to ordinary
+    outputs."""
+    print(f"exact small M={M} K={K} N={N} grow={grow}", flush=True)
+    signs, flags, lo, hi = _weight(K, N, 980 + N)
+    lo, hi = lo * np.float32(grow), hi * np.float32(grow)
+    A = P.gen_activations(SEED, 981 + M, M, K)
+    for r, scale in enumerate((1e-30, 1e-32, 1e-33, 1e-34, 1e-35, 1e-36, 1e-37, 1e-38, 1e-40, 1e-44)):
+        A[r] *= np.float32(scale)
+    A[10] *= np.float32(1e-38)
+    A[10, K // 3] = 1.0            # outputs whose weight there is 0 are made of the small values alone
+    A[11, ::7] *= np.float32(1e-37)
+    A[12] = 0.0
+    A[13, 1:] = 0.0
+    A[13, 0] = np.float32(1.4e-45)
+    A[14, 9:] = 0.0
+    if grow == 1.0:                # sums of halves overflow (3 of 1.6e38); those of products do not (9 x 3.2e38 x hi)
+        A[14, :9] = np.where(A[14, :9] < 0, np.float32(-3.2e38), np.float32(3.2e38))
+        assert 9 * 3.2e38 * float(hi.max()) < 3.4e38
+    got = P.fvb_gemm("exact", A, P.FvWeight(signs, flags, lo, hi, K, N)).astype(np.float64)
+    w = _expand64(signs, flags, lo, hi, N)
+    ref, mag = A.astype(np.float64) @ w, np.abs(A.astype(np.float64)) @ np.abs(w)
+    bad = np.abs(got - ref) > (K + 8) * (2.0 ** -24 * mag + 2.0 ** -149)
+    assert not bad.any(), f"rows {np.unique(np.argwhere(bad)[:, 0])[:16]}"
+
+
 def test_exact_code3_and_infinite_columns(monkeypatch):
     """Weights the plane kernels cannot hold (a code 3, an infinite hi) take the fmaf chain: its bits."""
     K, N, M = 128, 64, 40
