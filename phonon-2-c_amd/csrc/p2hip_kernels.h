@@ -3046,7 +3046,7 @@ __device__ __forceinline__ v4f xs_complete(const ExactArgs &g, int m, int n, v4f
  *     place c ^ (r % 16), so the operand reads below are free of bank conflicts); no barrier, each wave reads only its
  *     own slot: loads straight into the matrix-core layout touch 16 rows × 64 bytes per instruction, and the lines
  *     per instruction, not the bytes, set their pace.
- *   else: loads into registers in the matrix-core layout, units double-buffered.
+ *   else: loads into registers in the matrix-core layout, double-buffered.
  * VEC: K % 4 == 0, lda % 4 == 0 and A 16-byte aligned. */
 template <int FM, int FN, bool VEC, bool STAGED = false>
 __global__ __launch_bounds__(256, 2) void gemm_xf(ExactArgs g)
@@ -3176,8 +3176,8 @@ __global__ __launch_bounds__(256, 2) void gemm_xf(ExactArgs g)
             mma_step(0, 1, x);
         }
         __syncthreads();   /* every wave is done with its slots: the partial tiles reuse the area */
-    } else {
-        /* units double-buffered in registers: unit u + 1 loads while unit u is expanded and multiplied */
+    } else if constexpr (FM == 1) {
+        /* units double-buffered in registers: unit u + 1 loads while unit u is split and multiplied */
         float x[2][2][FM][16];
         auto load_unit = [&](int buf, int u) __attribute__((always_inline)) {
             load_records(buf, u);
@@ -3197,6 +3197,31 @@ __global__ __launch_bounds__(256, 2) void gemm_xf(ExactArgs g)
             if (u + 1 >= u_end) break;
             if (u + 2 < u_end) load_unit(0, u + 2);
             mma_unit(1);
+        }
+    } else {
+        /* 32 rows: steps double-buffered, the records a unit ahead. Two units of rows are 128 registers and spilled: K
+         * = 1001, N = 2048, M = 1000 73.3 against 59.2 µs, M = 4100 256 against 221; for 16 rows whole units are the
+         * faster (M = 375 21.5 against 24.2). */
+        float x[2][FM][16];
+        auto load_step = [&](int s, int u) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < FM; j++) load_x(j, 128 * u + 64 * s + 16 * grp, x[s][j]);
+        };
+        if (u_begin < u_end) {
+            load_records(0, u_begin);
+            load_step(0, u_begin);
+        }
+        for (int u = u_begin; u < u_end; u++) {
+            const int next = min(u + 1, u_end - 1);
+            load_step(1, u);
+            load_records(1, next);
+            mma_step(0, 0, x[0]);
+            load_step(0, next);
+            mma_step(0, 1, x[1]);
+#pragma unroll
+            for (int i = 0; i < FN; i++)
+#pragma unroll
+                for (int d = 0; d < 4; d++) r[0][i][d] = r[1][i][d];
         }
     }
 #pragma unroll

@@ -655,6 +655,24 @@ def test_exact_staged_rows_match_register_path(monkeypatch, M, K, N, lda, ldc, t
     _assert_exact(got[rows, :N], ref)
 
 
+@pytest.mark.parametrize("M,K,N,lda", [(75, 1001, 208, 1003), (37, 131, 80, 131), (40, 2052, 64, 2052), (33, 65, 16, 68),
+                                       (1030, 129, 2064, 129)])
+def test_exact_register_path_tiles_same_bits(monkeypatch, M, K, N, lda):
+    """Rows in registers (K or lda that the staged rows do not take): 32 x 64 tiles, whose steps are double-buffered,
+    against 16 x 16, whose units are, with odd numbers of units, a cut last unit and NaN past K; and the oracle."""
+    print(f"exact registers M={M} K={K} N={N} lda={lda}", flush=True)
+    signs, flags, lo, hi = _weight(K, N, 990 + K)
+    w = P.FvWeight(signs, flags, lo, hi, K, N)
+    A = np.full((M, lda), np.nan, np.float32)
+    A[:, :K] = P.gen_activations(SEED, 991 + M, M, K)
+    got = {}
+    for tile in (64, 1616):
+        monkeypatch.setenv("P2H_XF_TILE", str(tile))
+        got[tile] = P.fvb_gemm("exact", A, w)
+    assert _bits_equal(got[64], got[1616])
+    _assert_exact(got[64][:40], O.sgemm_fvb("exact", A[:40, :K].copy(), signs, flags, lo, hi, N))
+
+
 @pytest.mark.parametrize("M,K,N", [(2050, 100, 2064), (1090, 1156, 4096), (4099, 64, 1040), (2049, 192, 2048),
                                     (6000, 640, 704), (37, 200, 80), (130, 1024, 208), (9, 100, 32)])
 def test_exact_split_rows(monkeypatch, M, K, N):

@@ -99,3 +99,36 @@ def test_layer_norm_entries_reject_overlapping_rows():
     # the rows right after X do not overlap: the call passes those checks and stops at the next one (an invalid ldq)
     rc = ln2(X + 4 * D * M, D, D, ldq=1000)
     assert rc == -1 and "ldq" in P.last_error(), (rc, P.last_error())
+
+
+def _kernel_metadata(so):
+    """{kernel name: its metadata} of the gfx950 code objects inside a library built here: the AMDGPU metadata note
+    (type 32, MessagePack) of every embedded ELF of machine 224."""
+    import struct
+
+    import msgpack
+    data, out, at = open(so, "rb").read(), {}, 0
+    while (at := data.find(b"\x7fELF", at + 1)) > 0:
+        if struct.unpack_from("<H", data, at + 18)[0] != 224:
+            continue
+        shoff, shsize, shnum = (struct.unpack_from(f, data, at + o)[0] for f, o in (("<Q", 40), ("<H", 58), ("<H", 60)))
+        for s in range(shnum):
+            kind, _, _, off, size = struct.unpack_from("<IQQQQ", data, at + shoff + s * shsize + 4)
+            pos, end = at + off, at + off + size
+            while kind == 7 and pos < end:
+                namesz, descsz, ntype = struct.unpack_from("<III", data, pos)
+                desc = pos + 12 + (namesz + 3) // 4 * 4
+                if ntype == 32:
+                    note = msgpack.unpackb(data[desc:desc + descsz])
+                    out.update({k[".name"]: k for k in note["amdhsa.kernels"]})
+                pos = desc + (descsz + 3) // 4 * 4
+    return out
+
+
+def test_exact_kernels_do_not_spill():
+    """The exact route's matrix-core kernels keep everything in registers: two whole units of 32 rows held in them
+    spilled (200 bytes a lane, 8 % slower than the kernel before it at K = 1001 and a third at K = 2052)."""
+    kernels = {n: k for n, k in _kernel_metadata(P.HIP_SO).items() if "gemm_xf" in n or "gemm_xs" in n}
+    assert len(kernels) >= 6, sorted(kernels)
+    spills = {n: k[".private_segment_fixed_size"] for n, k in kernels.items() if k[".private_segment_fixed_size"]}
+    assert not spills, spills
