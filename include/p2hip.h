@@ -196,12 +196,15 @@ int p2h_fvb_gemm_q8a_grouped(int mode, int M, int N, int K, float alpha, const s
  * kernel adds them (exact) and folds the blocks in order, so results do not depend on the split. Calls sharing a
  * workspace must be stream-ordered. */
 size_t p2h_fvb_q8a_workspace_bytes(int mode, int M, int N, int K);
-/* The tile and split p2h_fvb_gemm_q8a chooses for a shape, as text (per thread; valid until the next call). */
+/* The tile and split p2h_fvb_gemm_q8a chooses for a shape, or in P2H_EXACT the kernel and tile p2h_fvb_gemm chooses for
+ * contiguous rows, as text (per thread; valid until the next call). */
 const char *p2h_fvb_plan(int mode, int M, int N, int K, int with_workspace);
 
 /* C = alpha · A · W + beta · C on fp32 A (p2_sgemm_fvb, blas.c:1481-1499): the int8 modes quantise A into the
- * workspace (at least p2h_fvb_workspace_bytes) and run p2h_fvb_gemm_q8a; P2H_EXACT (or K % 4 != 0) runs the fp32 expansion route, whose per-output
- * fmaf chain over k = 0..K-1 is the reference's exact kernel (blas.c:155-186, 929-987). */
+ * workspace (at least p2h_fvb_workspace_bytes) and run p2h_fvb_gemm_q8a; P2H_EXACT (or K % 4 != 0) multiplies the fp32
+ * rows by the weights' fp32 values, to within fp32 rounding of the reference's exact kernel, a per-output fmaf chain
+ * over k = 0..K-1 (blas.c:155-186, 929-987; P2H_EXACT_CHAIN=1 runs that chain, its bits). In every mode a row's outputs
+ * are the same bits whatever M is. */
 int    p2h_fvb_gemm(int mode, int M, int N, int K, float alpha, const float *dA, int lda, const P2hWeight *w,
                     float beta, float *dC, int ldc, void *workspace, size_t workspace_bytes, void *stream);
 size_t p2h_fvb_workspace_bytes(int mode, int M, int N, int K);

@@ -1378,6 +1378,34 @@ void launch_fv_cfg(const p2k::GemmArgs &g, const Plan &p, hipStream_t s)
     }
 }
 
+using XsL = p2k::XsGeo<2, 2, 2, 4>;   /* 64 × 128 */
+
+/* The exact route's kernel and tile, which change no bit of an output (XsCuts); vec: rows that allow 16-byte loads. */
+struct ExactPlan {
+    bool shared;   /* gemm_xs, else gemm_xf */
+    int bm, bn;
+};
+
+ExactPlan exact_plan(int M, int N, int K, bool vec)
+{
+    const long long cus = g_cus > 0 ? g_cus : 256;
+    auto tiles = [&](int bm, int bn) { return (long long)((N + bn - 1) / bn) * ((M + bm - 1) / bm); };
+    const int forced = switch_of(g_sw.xf_tile);
+    /* many rows: where gemm_xs' tiles fill its two workgroups per CU at least once (M = 6000, 1024 -> 4096: 228 against
+     * 272 µs for gemm_xf's best tile; at 192 tiles, M = 375, 28.4 against 21.9) */
+    if (forced == 0 && tiles(XsL::BM, XsL::BN) >= 2 * cus && K % 4 == 0 && K >= 64 && vec)
+        return {true, XsL::BM, XsL::BN};
+    /* measured with the weights from HBM, the same bits for every tile: 16 × 16 while those fit the CUs in one round
+     * (M = 38, 4096 -> 1024: 10.7 against 11.4 µs for 16 × 32), 16 × 32 up to three per CU (M = 125, 1024 -> 1024: 5.4
+     * against 5.8 and 6.9 for 16 × 16 and 16 × 64; M = 375, 4096 -> 1024: 25.4 against 33.8 and 27.9), 16 × 64 up to
+     * six (M = 125, 1024 -> 4096: 9.9 against 10.7 and 10.1 for 16 × 32 and 32 × 64), else 32 × 64 */
+    int bm = 16, bn = tiles(16, 16) <= cus ? 16 : tiles(16, 32) <= 3 * cus ? 32 : 64;
+    if (bn == 64 && tiles(16, 64) > 6 * cus) bm = 32;
+    if (forced == 32 || forced == 64) { bm = 32; bn = forced; }
+    if (forced == 1616 || forced == 1632 || forced == 1664) { bm = 16; bn = forced - 1600; }
+    return {false, bm, bn};
+}
+
 int check_split_ws(const char *who, const Plan &p, void *ws, size_t ws_bytes)
 {
     if (p.splits <= 1) return P2H_OK;
@@ -1394,6 +1422,14 @@ const char *p2h_fvb_plan(int mode, int M, int N, int K, int with_workspace)
 {
     static thread_local char buf[160];
     if (ensure_init() || M <= 0 || N <= 0 || K <= 0) return "";
+    if (mode == P2H_EXACT) {
+        const ExactPlan e = exact_plan(M, N, K, K % 4 == 0);
+        if (switch_of(g_sw.exact_chain) != 0) snprintf(buf, sizeof buf, "exact, fmaf chain");
+        else
+            snprintf(buf, sizeof buf, "exact, tile %dx%d, %s", e.bm, e.bn,
+                     e.shared ? "rows split once per workgroup" : "K split across the workgroup's waves");
+        return buf;
+    }
     Plan p = make_plan(mode == P2H_INT8 ? P2H_INT8 : P2H_INT8W, M, N, K, with_workspace != 0);
     if (is_small(p.cfg)) {
         const int a = xcd_rows_of(p, M, N);
@@ -1617,49 +1653,47 @@ static int launch_exact(int bkind, const p2k::ExactArgs &g0, hipStream_t s)
 
 namespace {
 
+template <int FM, int FN, int NW, int PPW, bool VEC, bool STAGED>
+void launch_xf_kernel(const p2k::ExactArgs &g, hipStream_t s)
+{
+    const dim3 grid((unsigned)((size_t)g.tiles_n * ((g.M + 16 * FM - 1) / (16 * FM)))), block(64 * NW);
+    hipLaunchKernelGGL((p2k::gemm_xf<FM, FN, NW, PPW, VEC, STAGED>), grid, block, 0, s, g);
+}
+
+/* Quarters of K in two pieces (K > 2048): eight waves for staged rows of 16 (4096 -> 1024: M = 38 7.8 against 10.1 µs
+ * for four waves of two pieces, M = 125 10.7 against 13.2); else four, since eight of more registers or LDS are one
+ * workgroup per CU (M = 2000 94.6 against 87.5 µs). */
 template <int FM, int FN>
 void launch_xf_tile(const p2k::ExactArgs &g, hipStream_t s)
 {
-    const dim3 grid((unsigned)((size_t)g.tiles_n * ((g.M + 16 * FM - 1) / (16 * FM)))), block(256);
     const bool vec = g.K % 4 == 0 && g.lda % 4 == 0 && aligned(g.A, 16);
     const bool staged = vec && g.K % 128 == 0 && switch_of(g_sw.xf_staged) != 0;
-    if (staged) hipLaunchKernelGGL((p2k::gemm_xf<FM, FN, true, true>), grid, block, 0, s, g);
-    else if (vec) hipLaunchKernelGGL((p2k::gemm_xf<FM, FN, true>), grid, block, 0, s, g);
-    else hipLaunchKernelGGL((p2k::gemm_xf<FM, FN, false>), grid, block, 0, s, g);
+    const bool two = p2k::XsCuts(g.units).two();
+    if (staged && two) launch_xf_kernel<FM, FN, FM == 1 ? 8 : 4, FM == 1 ? 1 : 2, true, true>(g, s);
+    else if (staged) launch_xf_kernel<FM, FN, 4, 1, true, true>(g, s);
+    else if (vec && two) launch_xf_kernel<FM, FN, 4, 2, true, false>(g, s);
+    else if (vec) launch_xf_kernel<FM, FN, 4, 1, true, false>(g, s);
+    else if (two) launch_xf_kernel<FM, FN, 4, 2, false, false>(g, s);
+    else launch_xf_kernel<FM, FN, 4, 1, false, false>(g, s);
 }
-
-using XsL = p2k::XsGeo<2, 2, 2, 4>;   /* 64 × 128 */
 
 int launch_xf(const p2k::ExactArgs &g0, hipStream_t s)
 {
     p2k::ExactArgs g = g0;
-    const long long cus = g_cus > 0 ? g_cus : 256;
-    auto tiles = [&](int bm, int bn) { return (long long)((g.N + bn - 1) / bn) * ((g.M + bm - 1) / bm); };
-    const int forced = switch_of(g_sw.xf_tile);
-    /* many rows: where gemm_xs' tiles fill its two workgroups per CU at least once (M = 6000, 1024 -> 4096: 228 against
-     * 272 µs for gemm_xf's best tile; at 192 tiles, M = 375, 28.4 against 21.9) */
-    if (forced == 0 && tiles(XsL::BM, XsL::BN) >= 2 * cus && g.K % 4 == 0 && g.K >= 64 && g.lda % 4 == 0 &&
-        aligned(g.A, 16)) {
-        g.tiles_n = (g.N + XsL::BN - 1) / XsL::BN;
-        const dim3 grid((unsigned)(8 * ((tiles(XsL::BM, XsL::BN) + 7) / 8))), block(XsL::NT);
+    const ExactPlan p = exact_plan(g.M, g.N, g.K, g.lda % 4 == 0 && aligned(g.A, 16));
+    g.tiles_n = (g.N + p.bn - 1) / p.bn;
+    if (p.shared) {
+        const long long tiles = (long long)g.tiles_n * ((g.M + p.bm - 1) / p.bm);
+        const dim3 grid((unsigned)(8 * ((tiles + 7) / 8))), block(XsL::NT);
         if (g.K % 64 == 0) hipLaunchKernelGGL((p2k::gemm_xs<XsL, false>), grid, block, 0, s, g);
         else hipLaunchKernelGGL((p2k::gemm_xs<XsL, true>), grid, block, 0, s, g);
         HIPCHK(hipGetLastError());
         return P2H_OK;
     }
-    /* measured with the weights from HBM, the same bits for every tile: 16 × 16 while those fit the CUs in one round
-     * (M = 38, 4096 -> 1024: 10.7 against 11.4 µs for 16 × 32), 16 × 32 up to three per CU (M = 125, 1024 -> 1024: 5.4
-     * against 5.8 and 6.9 for 16 × 16 and 16 × 64; M = 375, 4096 -> 1024: 25.4 against 33.8 and 27.9), 16 × 64 up to
-     * six (M = 125, 1024 -> 4096: 9.9 against 10.7 and 10.1 for 16 × 32 and 32 × 64), else 32 × 64 */
-    int bm = 16, bn = tiles(16, 16) <= cus ? 16 : tiles(16, 32) <= 3 * cus ? 32 : 64;
-    if (bn == 64 && tiles(16, 64) > 6 * cus) bm = 32;
-    if (forced == 32 || forced == 64) { bm = 32; bn = forced; }
-    if (forced == 1616 || forced == 1632 || forced == 1664) { bm = 16; bn = forced - 1600; }
-    g.tiles_n = (g.N + bn - 1) / bn;
-    if (bm == 16 && bn == 16) launch_xf_tile<1, 1>(g, s);
-    else if (bm == 16 && bn == 32) launch_xf_tile<1, 2>(g, s);
-    else if (bm == 16) launch_xf_tile<1, 4>(g, s);
-    else if (bn == 64) launch_xf_tile<2, 4>(g, s);
+    if (p.bm == 16 && p.bn == 16) launch_xf_tile<1, 1>(g, s);
+    else if (p.bm == 16 && p.bn == 32) launch_xf_tile<1, 2>(g, s);
+    else if (p.bm == 16) launch_xf_tile<1, 4>(g, s);
+    else if (p.bn == 64) launch_xf_tile<2, 4>(g, s);
     else launch_xf_tile<2, 2>(g, s);
     HIPCHK(hipGetLastError());
     return P2H_OK;

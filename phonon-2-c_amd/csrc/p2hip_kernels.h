@@ -2931,8 +2931,8 @@ __global__ __launch_bounds__(256) void gemm_exact(ExactArgs g)
  * a plane is exact, the sums are fp32 as on the fp32 matrix cores, and 2·lo and 2·hi scale the two planes' sums at the
  * end: six bf16 matrix instructions (16 × 16 × 32) do the work of eight fp32 ones (16 × 16 × 4), each in half the
  * time. No value is rounded on the way in and a 32-k step rounds a sum three times instead of eight, so the outputs are
- * nearer to the 64-bit ones than the fp32 instructions' (relative error, K = 1024 and 4096): 1.2e-7 and 2.3e-7 for
- * gemm_xf, 1.6e-7 and 1.7e-7 for gemm_xs, against 2.3e-7 and 4.5e-7.
+ * nearer to the 64-bit ones than the fp32 instructions' (relative error, K = 1024 and 4096): 1.2e-7 and 1.7e-7 against
+ * 2.3e-7 and 4.5e-7.
  *   Outputs that come out infinite or NaN are summed again by a scalar chain of fmaf over the expanded weights
  * (xs_complete, slow): the planes' zeros make NaN of an infinity's parts, and sums of halves could overflow where those of
  * the real products do not.
@@ -2990,6 +2990,16 @@ __device__ __forceinline__ void decode_planes(uint32_t r, v8bf &lo, v8bf &hi)
     hi = __builtin_bit_cast(v8bf, make_uint4(wh[0], wh[1], wh[2], wh[3]));
 }
 
+/* How the exact route's sums are cut along K, for every kernel and tile, so that a row's outputs do not depend on how
+ * many rows are multiplied with it: quarters of `su` 128-row units, a quarter of more than four in two pieces (`half`
+ * units, an even number, and the rest). A piece is summed by the matrix instructions in order of k and scaled by lo and hi; the pieces
+ * are added in order of k (without the second cut the error at K = 4096 is 2.3e-7). */
+struct XsCuts {
+    int su, half;
+    __host__ __device__ __forceinline__ explicit XsCuts(int units) : su((units + 3) / 4), half(su > 4 ? (su + 3) / 4 * 2 : su) {}
+    __host__ __device__ __forceinline__ bool two() const { return half < su; }
+};
+
 /* What split8's parts leave out of a value (0 from 2^-110 up). */
 __device__ __forceinline__ float left_out(float x)
 {
@@ -3032,10 +3042,10 @@ __device__ __forceinline__ v4f xs_complete(const ExactArgs &g, int m, int n, v4f
 /* The exact-mode five-value GEMM (sgemm_fvb_exact, blas.c:929-987): C = beta·C + alpha·A·W with exact products on the
  * bf16 matrix cores (above), for up to a few hundred rows. The sum runs in a different order from the reference's
  * per-output fmaf chain (which gemm_exact keeps bit for bit), so outputs agree to fp32 rounding.
- * A workgroup of four waves owns a BM × BN tile and splits K among its waves, as gemm_fvs does: each wave streams its
- * units' weight records (the 4-bit selectors of fv_repack4) and fp32 rows and splits and decodes both in registers;
- * lane l takes k = 16·(l / 16) .. + 15 of a 64-row step, which is the record's own order. The four partial tiles meet
- * in LDS and are added in wave order.
+ * A workgroup owns a BM × BN tile and splits K among its NW waves, as gemm_fvs does, a wave to PPW pieces (XsCuts):
+ * each wave streams its units' weight records (the 4-bit selectors of fv_repack4) and fp32 rows and splits and decodes both in registers;
+ * lane l takes k = 16·(l / 16) .. + 15 of a 64-row step, which is the record's own order. The partial tiles
+ * meet in LDS and are added in wave order.
  * The fp32 rows reach the lanes in one of two ways, with the same matrix instructions in the same order (the same
  * bits). Against the fp32 matrix cores (the same tiles, weights from HBM): M = 375, 1024 → 4096 34.0 → 21.9 µs,
  * 4096 → 1024 37.8 → 25.4, 1024 → 1024 13.0 → 9.3; M = 125, 1024 → 4096 13.9 → 9.9; M = 38, 4096 → 1024
@@ -3048,25 +3058,28 @@ __device__ __forceinline__ v4f xs_complete(const ExactArgs &g, int m, int n, v4f
  *     per instruction, not the bytes, set their pace.
  *   else: loads into registers in the matrix-core layout, double-buffered.
  * VEC: K % 4 == 0, lda % 4 == 0 and A 16-byte aligned. */
-template <int FM, int FN, bool VEC, bool STAGED = false>
-__global__ __launch_bounds__(256, 2) void gemm_xf(ExactArgs g)
+template <int FM, int FN, int NW, int PPW, bool VEC, bool STAGED = false>
+__global__ __launch_bounds__(64 * NW, 2) void gemm_xf(ExactArgs g)
 {
     static_assert(!STAGED || VEC, "the staged rows are read as 16-byte chunks");
-    constexpr int NW = 4, NT = 64 * NW;
+    static_assert(NW * PPW == 4 || NW * PPW == 8, "a quarter of K is one piece or two");
+    constexpr int NT = 64 * NW;
     constexpr int BM = 16 * FM, BN = 16 * FN, PITCH = BN + 4, TILE = BM * PITCH;
     constexpr int ABUF = BM * 256;                    /* STAGED: one 64-row K stage of one wave, BM rows × 256 bytes */
     constexpr int NQ = BM / 4;                        /* STAGED: direct loads per stage, four rows each */
     constexpr int SMEM = (STAGED && NW * ABUF > 4 * NW * TILE) ? NW * ABUF : 4 * NW * TILE;   /* bytes */
-    __shared__ __attribute__((aligned(16))) int8_t smem[SMEM];   /* the partial tiles reuse the staging slots */
-    float *part = reinterpret_cast<float *>(smem);
+    /* the partial tiles reuse the staging slots, but for the first ones of PPW = 2 */
+    __shared__ __attribute__((aligned(16))) int8_t smem[SMEM + 4 * (PPW - 1) * NW * TILE];
+    float *part = reinterpret_cast<float *>(smem), *part1 = reinterpret_cast<float *>(smem + SMEM);
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, grp = lane >> 4;
     const int tile_n = blockIdx.x % g.tiles_n, tile_m = blockIdx.x / g.tiles_n;
     const int n0 = tile_n * BN, m0 = tile_m * BM;
     const int M = g.M, N = g.N, K = g.K, units = g.units;
-    const int su = (units + NW - 1) / NW;
-    const int nseg = (units + su - 1) / su;
-    const int u_begin = min(units, wave * su), u_end = min(units, u_begin + su);
+    const XsCuts cuts(units);
+    const int quarter = wave / (NW / 4) * cuts.su, mid = min(units, quarter + cuts.half);
+    const int w_begin = NW == 8 && (wave & 1) ? mid : min(units, quarter);
+    const int w_end = NW == 8 && !(wave & 1) ? mid : min(units, quarter + cuts.su);
 
     __shared__ int lowbits[BM];   /* 1: a row with values whose parts leave bits out */
     for (int c = tid; c < BM; c += NT) lowbits[c] = 0;
@@ -3131,8 +3144,44 @@ __global__ __launch_bounds__(256, 2) void gemm_xf(ExactArgs g)
             r[rb][i][0] = v.x; r[rb][i][1] = v.y; r[rb][i][2] = v.z; r[rb][i][3] = v.w;
         }
     };
+    /* this wave's sums of a piece: 2·lo and 2·hi (as the reference expands it) times the planes' */
+    auto put_piece = [&](float *area) __attribute__((always_inline)) {
+        int n_at = n0 + 4 * grp, at = wave * TILE + (lane & 15) * PITCH + 4 * grp;
+        if (PPW > 1) asm volatile("" : "+v"(n_at), "+v"(at));   /* made here, not held in registers through the loop */
+#pragma unroll
+        for (int i = 0; i < FN; i++) {
+            const int n = min(n_at + 16 * i, N - 4);
+            float lo[4], hi[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                lo[e] = g.lo[n + e];
+                hi[e] = 2.0f * __builtin_fmaf(1.0f, g.hi[n + e] - lo[e], lo[e]);
+                lo[e] *= 2.0f;
+            }
+#pragma unroll
+            for (int j = 0; j < FM; j++) {
+                v4f f;
+#pragma unroll
+                for (int e = 0; e < 4; e++) f[e] = __builtin_fmaf(lo[e], accL[i][j][e], hi[e] * accH[i][j][e]);
+                *reinterpret_cast<v4f *>(area + at + 16 * j * PITCH + 16 * i) = f;
+                accL[i][j] = accH[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+        }
+    };
+    /* the wave's pieces, each summed by multiply(first unit, end) */
+    auto each_piece = [&](auto &&multiply) __attribute__((always_inline)) {
+        if constexpr (PPW == 1) {
+            multiply(w_begin, w_end);
+        } else {
+#pragma unroll 1
+            for (int pc = 0; pc < 2; pc++) {
+                multiply(pc == 0 ? w_begin : mid, pc == 0 ? mid : w_end);
+                if (pc == 0) put_piece(part1);
+            }
+        }
+    };
     if constexpr (STAGED) {
-        /* stage st = 2·(u − u_begin) + s into this wave's slot; load q brings rows 4q .. 4q + 3, lane L filling place
+        /* step s of unit u into this wave's slot; load q brings rows 4q .. 4q + 3, lane L filling place
          * L % 16 of row 4q + L / 16 with that row's chunk (L % 16) ^ (row % 16) */
         const float *a_src[NQ];
 #pragma unroll
@@ -3141,13 +3190,11 @@ __global__ __launch_bounds__(256, 2) void gemm_xf(ExactArgs g)
             a_src[q] = g.A + (size_t)min(m0 + rr, M - 1) * g.lda + 4 * ((lane & 15) ^ (rr & 15));
         }
         int8_t *slot = smem + wave * ABUF;
-        const int n_st = 2 * (u_end - u_begin);
-        auto issue = [&](int st) __attribute__((always_inline)) {
-            const int u = u_begin + (st >> 1);
+        auto issue = [&](int u, int s) __attribute__((always_inline)) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   /* this wave's reads of the slot are complete */
 #pragma unroll
-            for (int q = 0; q < NQ; q++) dma_16(a_src[q] + 128 * u + 64 * (st & 1), slot + q * 1024);
-            if ((st & 1) == 0) load_records(0, u);
+            for (int q = 0; q < NQ; q++) dma_16(a_src[q] + 128 * u + 64 * s, slot + q * 1024);
+            if (s == 0) load_records(0, u);
         };
         float x[FM][16];
         auto read = [&]() __attribute__((always_inline)) {
@@ -3163,21 +3210,24 @@ __global__ __launch_bounds__(256, 2) void gemm_xf(ExactArgs g)
         };
         /* one slot per wave: step 1 loads while step 0 is multiplied (the barriers keep it so), the wait for step 0
          * is covered by the other waves of the CU */
-        for (int st = 0; st < n_st; st += 2) {
-            issue(st);        /* step 0 of the unit and its records */
-            wait_vm<0>();
-            read();
-            issue(st + 1);    /* step 1 */
-            __builtin_amdgcn_sched_barrier(0);
-            mma_step(0, 0, x);
-            __builtin_amdgcn_sched_barrier(0);
-            wait_vm<0>();
-            read();
-            mma_step(0, 1, x);
-        }
+        each_piece([&](int u_begin, int u_end) __attribute__((always_inline)) {
+            for (int u = u_begin; u < u_end; u++) {
+                issue(u, 0);      /* step 0 of the unit and its records */
+                wait_vm<0>();
+                read();
+                issue(u, 1);      /* step 1 */
+                __builtin_amdgcn_sched_barrier(0);
+                mma_step(0, 0, x);
+                __builtin_amdgcn_sched_barrier(0);
+                wait_vm<0>();
+                read();
+                mma_step(0, 1, x);
+            }
+        });
         __syncthreads();   /* every wave is done with its slots: the partial tiles reuse the area */
     } else if constexpr (FM == 1) {
-        /* units double-buffered in registers: unit u + 1 loads while unit u is split and multiplied */
+        /* units double-buffered in registers: unit u + 1 loads while unit u is split and multiplied. The pieces are cut
+         * inside the loop (the first has an even number of units): a loop over them took 40 registers more. */
         float x[2][2][FM][16];
         auto load_unit = [&](int buf, int u) __attribute__((always_inline)) {
             load_records(buf, u);
@@ -3190,14 +3240,16 @@ __global__ __launch_bounds__(256, 2) void gemm_xf(ExactArgs g)
             mma_step(buf, 0, x[buf][0]);
             mma_step(buf, 1, x[buf][1]);
         };
-        if (u_begin < u_end) load_unit(0, u_begin);
-        for (int u = u_begin; u < u_end; u += 2) {
-            if (u + 1 < u_end) load_unit(1, u + 1);
+        if (w_begin < w_end) load_unit(0, w_begin);
+        for (int u = w_begin; u < w_end; u += 2) {
+            if (u + 1 < w_end) load_unit(1, u + 1);
+            if (PPW == 2 && u == mid) put_piece(part1);
             mma_unit(0);
-            if (u + 1 >= u_end) break;
-            if (u + 2 < u_end) load_unit(0, u + 2);
+            if (u + 1 >= w_end) break;
+            if (u + 2 < w_end) load_unit(0, u + 2);
             mma_unit(1);
         }
+        if (PPW == 2 && mid >= w_end) put_piece(part1);   /* cut short: the second piece is empty */
     } else {
         /* 32 rows: steps double-buffered, the records a unit ahead. Two units of rows are 128 registers and spilled: K
          * = 1001, N = 2048, M = 1000 73.3 against 59.2 µs, M = 4100 256 against 221; for 16 rows whole units are the
@@ -3207,47 +3259,29 @@ __global__ __launch_bounds__(256, 2) void gemm_xf(ExactArgs g)
 #pragma unroll
             for (int j = 0; j < FM; j++) load_x(j, 128 * u + 64 * s + 16 * grp, x[s][j]);
         };
-        if (u_begin < u_end) {
-            load_records(0, u_begin);
-            load_step(0, u_begin);
+        if (w_begin < w_end) {
+            load_records(0, w_begin);
+            load_step(0, w_begin);
         }
-        for (int u = u_begin; u < u_end; u++) {
-            const int next = min(u + 1, u_end - 1);
-            load_step(1, u);
-            load_records(1, next);
-            mma_step(0, 0, x[0]);
-            load_step(0, next);
-            mma_step(0, 1, x[1]);
+        each_piece([&](int u_begin, int u_end) __attribute__((always_inline)) {
+            for (int u = u_begin; u < u_end; u++) {
+                const int next = min(u + 1, w_end - 1);
+                load_step(1, u);
+                load_records(1, next);
+                mma_step(0, 0, x[0]);
+                load_step(0, next);
+                mma_step(0, 1, x[1]);
 #pragma unroll
-            for (int i = 0; i < FN; i++)
+                for (int i = 0; i < FN; i++)
 #pragma unroll
-                for (int d = 0; d < 4; d++) r[0][i][d] = r[1][i][d];
-        }
+                    for (int d = 0; d < 4; d++) r[0][i][d] = r[1][i][d];
+            }
+        });
     }
 #pragma unroll
     for (int j = 0; j < FM; j++)
         if (low[j] & 0xffffu) lowbits[16 * j + (lane & 15)] = 1;
-    if (wave < nseg) {   /* this wave's sums: 2·lo and 2·hi (as the reference expands it) times the planes' */
-        float *dst = part + wave * TILE;
-#pragma unroll
-        for (int i = 0; i < FN; i++) {
-            const int n = min(n0 + 16 * i + 4 * grp, N - 4);
-            float lo[4], hi[4];
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                lo[e] = g.lo[n + e];
-                hi[e] = 2.0f * __builtin_fmaf(1.0f, g.hi[n + e] - lo[e], lo[e]);
-                lo[e] *= 2.0f;
-            }
-#pragma unroll
-            for (int j = 0; j < FM; j++) {
-                v4f f;
-#pragma unroll
-                for (int e = 0; e < 4; e++) f[e] = __builtin_fmaf(lo[e], accL[i][j][e], hi[e] * accH[i][j][e]);
-                *reinterpret_cast<v4f *>(dst + (16 * j + (lane & 15)) * PITCH + 16 * i + 4 * grp) = f;
-            }
-        }
-    }
+    put_piece(part);
     __syncthreads();
 
     constexpr int TPR = BN / 4, RPP = NT / TPR;
@@ -3256,8 +3290,13 @@ __global__ __launch_bounds__(256, 2) void gemm_xf(ExactArgs g)
     for (int row = tid / TPR; row < BM; row += RPP) {
         const int m = m0 + row;
         if (m >= M) break;
-        v4f sum = *reinterpret_cast<const v4f *>(part + row * PITCH + 4 * cq);
-        for (int sg = 1; sg < nseg; sg++) sum += *reinterpret_cast<const v4f *>(part + sg * TILE + row * PITCH + 4 * cq);
+        v4f sum = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int sg = 0; sg < NW; sg++) {
+            const int at = sg * TILE + row * PITCH + 4 * cq;
+            if (PPW == 2) sum += *reinterpret_cast<const v4f *>(part1 + at);
+            sum += *reinterpret_cast<const v4f *>(part + at);
+        }
         sum = xs_complete(g, m, n, sum, lowbits[row] != 0);
         float *cp = g.C + (size_t)m * g.ldc + n;
         if (n + 3 < N && (reinterpret_cast<uintptr_t>(cp) & 15) == 0) {   /* one 16-byte store */

@@ -7,7 +7,6 @@
 
 namespace p2k {
 
-constexpr int kXsSeg = 512;   /* K rows per segment: its sums are folded into the running outputs, then start again */
 template <int WM_, int WN_, int FM_, int FN_>
 struct XsGeo {
     static constexpr int WM = WM_, WN = WN_, FM = FM_, FN = FN_;
@@ -22,8 +21,8 @@ struct XsGeo {
  * all its waves (in gemm_xf every wave splits what it reads, and the split's VALU work bounds it), so the matrix cores
  * have 96 instructions a step for a thread's 16 split values. Waves are WM × WN over the tile, each FM row groups by
  * FN column groups; rows are two steps ahead in registers and one in the two-slot LDS ring (a barrier a step), records
- * a unit ahead in registers. Every 512 rows of K the planes' sums are folded into running outputs, which keeps the
- * additions' rounding below the fp32 instructions' (1.7e-7 against 4.5e-7 at K = 4096). 64 × 128, two workgroups per
+ * a unit ahead in registers. At the end of each piece of K (XsCuts) the planes' sums are folded into running outputs,
+ * which gives gemm_xf's bits. 64 × 128, two workgroups per
  * CU: M = 6000, 4096 → 1024 421 → 220 µs and 1024 → 4096 438 → 228, 1.37 PFLOP/s of bf16 products (a loop of nothing
  * but these matrix instructions runs at 1.7–1.8 on this card, power-bound); 48 × 128 was 228 / 230, 64 × 64 251 / 254,
  * and 96 × 128 spilled (289 / 300). */
@@ -167,8 +166,14 @@ __global__ __launch_bounds__(G::NT, 2) void gemm_xs(ExactArgs g)
     load_a(0, av[0]);
     load_a(1, av[1]);
     put_a(0, 0, av[0]);
-    constexpr int SEG_UNITS = kXsSeg / 128;
+    const XsCuts cuts(units);
+    int cut = cuts.half, piece = cuts.half;   /* the unit before which the next piece starts; this piece's length */
     for (int u = 0; u < units; u++) {
+        if (u == cut) {
+            fold();
+            if (cuts.half < cuts.su) piece = cuts.su - piece;
+            cut += piece;
+        }
         rec_of(u + 1, nrec);
         load_a(2 * u + 2, av[0]);
         lds_barrier();   /* slot 0 is written (and slot 1 read out) by every wave */
@@ -180,7 +185,6 @@ __global__ __launch_bounds__(G::NT, 2) void gemm_xs(ExactArgs g)
         put_a(2 * u + 2, 0, av[0]);   /* past the last unit: unused */
 #pragma unroll
         for (int i = 0; i < FN; i++) rec[i] = nrec[i];
-        if ((u + 1) % SEG_UNITS == 0 && u + 1 < units) fold();
     }
     fold();
 #pragma unroll

@@ -611,7 +611,7 @@ def test_exact_full_size_sampled_rows(monkeypatch, M, K, N):
 @pytest.mark.parametrize("M,K,N", [(375, 4096, 1024), (38, 1024, 4096), (130, 1024, 208), (9, 4096, 64)])
 def test_exact_tiles_same_bits(monkeypatch, M, K, N):
     """Every output of the exact route's matrix-core kernel is summed in the same order whatever the tile (each MFMA
-    step covers the same four K rows, and the waves' K segments meet in wave order), so all five tiles give the same
+    covers the same 32 K rows, and the waves' pieces of K meet in order of k), so all five tiles give the same
     bits; the planner's choice among them is a matter of speed only."""
     signs, flags, lo, hi = _weight(K, N, 940 + M + N)
     w = P.FvWeight(signs, flags, lo, hi, K, N)
@@ -621,6 +621,25 @@ def test_exact_tiles_same_bits(monkeypatch, M, K, N):
     for tile in (32, 64, 1616, 1632, 1664):
         monkeypatch.setenv("P2H_XF_TILE", str(tile))
         assert _bits_equal(P.fvb_gemm("exact", A, w, alpha=0.7, beta=1.0, C0=C0), base), f"tile {tile}"
+
+
+@pytest.mark.parametrize("M,K,N", [(2050, 1024, 2064), (2050, 4096, 2064), (2049, 2052, 2048), (1100, 1156, 4096),
+                                    (2050, 64, 2064), (2050, 700, 2064), (1100, 4352, 4096)])
+def test_exact_rows_same_bits_any_count(M, K, N):
+    """A row's exact outputs do not depend on how many rows the call has: many rows (gemm_xs, which adds its pieces of
+    K into running outputs) against the same rows in smaller calls (gemm_xf, whose waves take a quarter of K each);
+    whole, cut and empty second pieces."""
+    few = (1, 38, 130, 375)
+    print(f"exact any count M={M} K={K} N={N} {P.plan('exact', M, N, K)}", flush=True)
+    assert "once per workgroup" in P.plan("exact", M, N, K)
+    assert all("workgroup's waves" in P.plan("exact", m, N, K) for m in few)
+    w = P.FvWeight(*_weight(K, N, 945 + K), K, N)
+    A = P.gen_activations(SEED, 946 + K, M, K)
+    A[3] *= np.float32(1e-37)
+    C0 = np.random.default_rng(K).standard_normal((M, N)).astype(np.float32)
+    all_rows = P.fvb_gemm("exact", A, w, alpha=0.7, beta=1.0, C0=C0)
+    for m in few:
+        assert _bits_equal(P.fvb_gemm("exact", A[:m], w, alpha=0.7, beta=1.0, C0=C0[:m]), all_rows[:m]), f"{m} rows"
 
 
 @pytest.mark.parametrize("M,K,N,lda,ldc,tile", [
