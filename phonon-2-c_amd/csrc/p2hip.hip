@@ -13,6 +13,7 @@
 #include <cstdlib>
 #include <climits>
 #include <atomic>
+#include <type_traits>
 #include <mutex>
 #include <vector>
 
@@ -1180,6 +1181,8 @@ using G3264 = p2k::Geo<32, 64, 2, 2, 256>;   /* int8-table GEMMs: K <= 1024 when
 struct Plan {
     int cfg, splits, split_rows, tiles_m, tiles_n;
     size_t part_bytes;
+    bool rb;         /* runs on gemm_fv_rb (weight records in registers) */
+    bool silu;       /* the kernel can apply SiLU as it stores C */
 };
 
 /* Tile and K split of a five-value call. A split is a whole number of 128-row units inside one 1024-row fold block;
@@ -1258,6 +1261,9 @@ Plan make_plan(int mode, int M, int N, int K, bool can_split)
     }
     const size_t planes = mode == P2H_INT8 ? 2 : 1;
     p.part_bytes = p.splits > 1 ? align_up(planes * p.splits * (size_t)M * N * 4, 256) : 0;
+    p.rb = (cfg == FV_W6 || cfg == FV_WK) && switch_of(g_sw.records_in_regs) != 0;
+    /* not the 96 × 256 tile with running sums (K > 1024, forced only): with the SiLU it spilled 165 registers */
+    p.silu = is_small(cfg) || (p.rb && !(cfg == FV_W6 && K > p2k::kFoldRows));
     return p;
 }
 
@@ -1298,22 +1304,21 @@ p2k::GemmArgs gemm_args(int M, int N, int K, float alpha, float beta, const sign
     return g;
 }
 
-/* the plan runs on gemm_fv_rb */
-bool records_in_regs(const Plan &p)
-{
-    return (p.cfg == FV_W6 || p.cfg == FV_WK) && switch_of(g_sw.records_in_regs) != 0;
-}
-
 /* the large-M tiles: unsplit, two workgroups per CU, 4-bit records (in registers, or through the LDS ring with the
  * activation rows), staged output rows */
 template <class G>
 void launch_fv_large(const p2k::GemmArgs &g, const Plan &p, hipStream_t s)
 {
     const dim3 grid((unsigned)((size_t)p.tiles_m * p.tiles_n)), block(G::NT);
-    if (switch_of(g_sw.records_in_regs)) {
+    if (p.rb) {
         const bool multi = g.K > p2k::kFoldRows;
-        if (multi && g.act) hipLaunchKernelGGL((p2k::gemm_fv_rb<G, true, true>), grid, block, 0, s, g);
-        else if (multi) hipLaunchKernelGGL((p2k::gemm_fv_rb<G, true, false>), grid, block, 0, s, g);
+        if constexpr (std::is_same<G, FvWK>::value) {   /* of the two, the one with SiLU and running sums (Plan::silu) */
+            if (multi && g.act) {
+                hipLaunchKernelGGL((p2k::gemm_fv_rb<G, true, true>), grid, block, 0, s, g);
+                return;
+            }
+        }
+        if (multi) hipLaunchKernelGGL((p2k::gemm_fv_rb<G, true, false>), grid, block, 0, s, g);
         else if (g.act) hipLaunchKernelGGL((p2k::gemm_fv_rb<G, false, true>), grid, block, 0, s, g);
         else hipLaunchKernelGGL((p2k::gemm_fv_rb<G, false, false>), grid, block, 0, s, g);
         return;
@@ -1349,33 +1354,44 @@ void launch_fvs(const p2k::GemmArgs &g, const Plan &p, hipStream_t s)
                        g);
 }
 
+/* The kernel of the plan's tile, for which its grid is sized. False, and nothing launched, where the mode has none:
+ * make_plan gives the two-plane mode no such tile. */
 template <int MODE>
-void launch_fv_cfg(const p2k::GemmArgs &g, const Plan &p, hipStream_t s)
+bool launch_fv_cfg(const p2k::GemmArgs &g, const Plan &p, hipStream_t s)
 {
     switch (p.cfg) {
     case FV_SS: launch_fvs<SmS, MODE>(g, p, s); break;
     case FV_SW: case FV_SD: case FV_SS8: case FV_SW8: case FV_SQ: case FV_SQ8: case FV_SR8:
-        if (MODE != p2k::MODE_INT8W) { launch_fvs<SmS, MODE>(g, p, s); break; }   /* make_plan maps int8 away */
-        with_small_geo(p.cfg, [&](auto geo) { launch_fvs<decltype(geo), p2k::MODE_INT8W>(g, p, s); });
-        break;
+        if (MODE != p2k::MODE_INT8W) return false;
+        return with_small_geo(p.cfg, [&](auto geo) { launch_fvs<decltype(geo), p2k::MODE_INT8W>(g, p, s); });
     case FV_T: launch_fv<FvT, MODE>(g, p, s); break;
     case FV_S: launch_fv<FvS, MODE>(g, p, s); break;
     case FV_M: launch_fv<FvM, MODE>(g, p, s); break;
     case FV_T8: launch_fv<FvT8, MODE>(g, p, s); break;
     case FV_S8: launch_fv<FvS8, MODE>(g, p, s); break;
     case FV_T6: launch_fv<FvT6, MODE>(g, p, s); break;
-    case FV_W6: if (MODE == p2k::MODE_INT8W) { launch_fv_large<FvW6>(g, p, s); break; } /* fall through */
+    case FV_W6:
+        if (MODE != p2k::MODE_INT8W) return false;
+        launch_fv_large<FvW6>(g, p, s);
+        break;
     case FV_WK:
-        if (MODE == p2k::MODE_INT8W) { launch_fv_large<FvWK>(g, p, s); break; }
-        {   /* the two-plane mode: one fold block (make_plan) */
+        if (MODE == p2k::MODE_INT8W) {
+            launch_fv_large<FvWK>(g, p, s);
+        } else {   /* the two-plane mode: one fold block, records in registers */
+            if (!p.rb || g.K > p2k::kFoldRows) return false;
             const dim3 grid((unsigned)((size_t)p.tiles_m * p.tiles_n)), block(FvWK::NT);
             if (g.act) hipLaunchKernelGGL((p2k::gemm_fv_rb<FvWK, false, true, p2k::MODE_INT8>), grid, block, 0, s, g);
             else hipLaunchKernelGGL((p2k::gemm_fv_rb<FvWK, false, false, p2k::MODE_INT8>), grid, block, 0, s, g);
         }
         break;
-    case FV_X: if (MODE == p2k::MODE_INT8W) { launch_fv<FvX, p2k::MODE_INT8W>(g, p, s); break; } /* fall through */
-    default: launch_fv<FvL, MODE>(g, p, s); break;
+    case FV_X:
+        if (MODE != p2k::MODE_INT8W) return false;
+        launch_fv<FvX, p2k::MODE_INT8W>(g, p, s);
+        break;
+    case FV_L: launch_fv<FvL, MODE>(g, p, s); break;
+    default: return false;
     }
+    return true;
 }
 
 using XsL = p2k::XsGeo<2, 2, 2, 4>;   /* 64 × 128 */
@@ -1442,7 +1458,7 @@ const char *p2h_fvb_plan(int mode, int M, int N, int K, int with_workspace)
         snprintf(buf, sizeof buf, "tile %dx%d, %d split%s of %d rows%s%s", kFvBM[p.cfg], kFvBN[p.cfg], p.splits,
                  p.splits > 1 ? "s" : "", p.split_rows,
                  p.splits > 1 ? " + fold" : (K > p2k::kFoldRows ? ", folds in registers" : ""),
-                 records_in_regs(p) ? ", weight records in registers" : "");
+                 p.rb ? ", weight records in registers" : "");
     return buf;
 }
 
@@ -1513,15 +1529,17 @@ static int fvb_gemm_q8a(int mode, int M, int N, int K, float alpha, const signed
         g.warm = next->rec4;
         g.warm_lines = (int)std::min<size_t>((bytes + 127) / 128, 0x7fffffff);
     }
-    const bool silu_here = silu && (is_small(p.cfg) || records_in_regs(p));
+    const bool silu_here = silu && p.silu;
     g.act = silu_here ? 1 : 0;
+    bool launched;
     if (mode == P2H_INT8W) {
         g.c1 = w->hi; g.c1_hi = 1;
-        launch_fv_cfg<p2k::MODE_INT8W>(g, p, s);
+        launched = launch_fv_cfg<p2k::MODE_INT8W>(g, p, s);
     } else {
         g.c1 = w->lo; g.c2 = w->hi;
-        launch_fv_cfg<p2k::MODE_INT8>(g, p, s);
+        launched = launch_fv_cfg<p2k::MODE_INT8>(g, p, s);
     }
+    if (!launched) return fail(P2H_E_ARG, "p2h_fvb_gemm_q8a: mode %d has no kernel for tile %d", mode, p.cfg);
     HIPCHK(hipGetLastError());
     if (silu && !silu_here) return p2h_silu((size_t)M * N, dC, s);
     return P2H_OK;

@@ -410,6 +410,18 @@ def test_q8a_silu_large_tiles(M, K, N):
     assert _bits_equal(got, ref)
 
 
+def test_q8a_silu_forced_wide_tile(monkeypatch):
+    """The 96 x 256 tile forced at K > 1024, which runs the SiLU as a pass of its own: the bits of GEMM then p2h_silu."""
+    M, K, N = 300, 1156, 528
+    print(f"q8a silu forced 96x256 M={M} K={K} N={N}", flush=True)
+    monkeypatch.setenv("P2H_TILE", "8")
+    assert P.plan("int8w", M, N, K).startswith("tile 96x256,")
+    q, sc = O.quant_rows(P.gen_activations(SEED, 1990, M, K))
+    w = P.FvWeight(*_weight(K, N, 1991), K, N)
+    got = P.fvb_gemm_q8a_silu("int8w", q, sc, w, alpha=0.7)
+    assert _bits_equal(got, P.silu(P.fvb_gemm_q8a("int8w", q, sc, w, alpha=0.7)))
+
+
 # ── several weights against the same quantised rows in one launch ─────────────────────────────────────────────────
 
 @pytest.mark.parametrize("mode", ["int8w", "int8"])
