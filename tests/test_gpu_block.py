@@ -394,6 +394,22 @@ def test_exact_epilogues_same_bits(monkeypatch, T):
     assert np.array_equal(fused.view(np.uint32), separate.view(np.uint32))
 
 
+def test_exact_epilogues_many_rows_same_bits(monkeypatch):
+    """The same where the up-projections have enough tiles for gemm_xs: its SiLU against a pass of its own."""
+    T = 1030
+    print(f"exact epilogues T={T} {P.plan('exact', T, 4096, 1024)}", flush=True)
+    assert "once per workgroup" in P.plan("exact", T, 4096, 1024)
+    sys.path.insert(0, HERE)
+    import refblock_child as RC
+    x, pe = RC.block_input(SEED, T)
+    blk = _device_block(SEED)
+    fused = blk.run("exact", x, pe)
+    monkeypatch.setenv("P2H_EXACT_EPILOGUE", "0")
+    separate = blk.run("exact", x, pe)
+    assert np.isfinite(fused).all()
+    assert np.array_equal(fused.view(np.uint32), separate.view(np.uint32))
+
+
 @pytest.mark.parametrize("mode,T", [("int8w", 375), ("int8", 375), ("int8w", 40)])
 def test_silu_epilogue_same_bits(monkeypatch, mode, T):
     """The int8 modes apply the feed-forward's SiLU in the up-projection's epilogue and quantise its rows with the

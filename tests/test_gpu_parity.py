@@ -364,11 +364,13 @@ def test_q8a_next_matches_q8a(mode, M, K, N, Kn, Nn, beta):
 # ── the feed-forward's SiLU in the up-projection's epilogue ───────────────────────────────────────────────────────
 
 @pytest.mark.parametrize("mode", ["int8w", "int8"])
-@pytest.mark.parametrize("M,K,N", [(375, 1024, 4096), (38, 1024, 4096), (375, 4096, 272), (2000, 1024, 1024)])
+@pytest.mark.parametrize("M,K,N", [(375, 1024, 4096), (38, 1024, 4096), (375, 4096, 272), (2000, 1024, 1024),
+                                    (1100, 1156, 272)])
 def test_q8a_silu_matches_gemm_then_silu(mode, M, K, N):
     """p2h_fvb_gemm_q8a_silu equals p2h_fvb_gemm_q8a followed by p2h_silu bit for bit: the small-M tiles and the
-    int8w large-M tiles apply silu_p2 as they store C; the two-plane mode at 2000 rows runs the SiLU kernel after
-    the GEMM."""
+    large-M tiles with records in registers apply silu_p2 as they store C; the two-plane mode beyond 1024 rows and
+    K = 1024 runs the SiLU kernel after the GEMM."""
+    assert ("registers" in P.plan(mode, M, N, K)) == (M > 1024 and (mode == "int8w" or K <= 1024))
     A = P.gen_activations(SEED, 1900 + M, M, K)
     q, sc = O.quant_rows(A)
     w = P.FvWeight(*_weight(K, N, 1910 + N), K, N)
@@ -384,6 +386,7 @@ def test_two_plane_records_in_registers(monkeypatch, M, K, N, beta):
     """The two-plane mode's 96 x 128 tiles with the records in registers: the bits of the 128 x 128 tiles
     (P2H_RECORDS_IN_REGISTERS=0), with cut row and column tiles, and of the SiLU after the GEMM."""
     print(f"two-plane M={M} K={K} N={N} beta={beta} {P.plan('int8', M, N, K)}", flush=True)
+    assert "weight records in registers" in P.plan("int8", M, N, K)
     A = P.gen_activations(SEED, 1970 + M, M, K)
     q, sc = O.quant_rows(A)
     w = P.FvWeight(*_weight(K, N, 1980 + N), K, N)
@@ -396,11 +399,28 @@ def test_two_plane_records_in_registers(monkeypatch, M, K, N, beta):
     assert _bits_equal(act, P.fvb_gemm_q8a_silu("int8", q, sc, w, alpha=0.7))
 
 
+@pytest.mark.parametrize("M,K,N,ldc", [(1030, 384, 272, 275), (1100, 640, 144, 145), (1501, 100, 528, 530)])
+@pytest.mark.parametrize("beta", [0.0, 1.0])
+def test_two_plane_records_in_registers_strides(monkeypatch, M, K, N, ldc, beta):
+    """The same with C's rows stored element by element (ldc not a multiple of 4) and odd numbers of 128-row units;
+    columns past N stay as they were."""
+    print(f"two-plane strides M={M} K={K} N={N} ldc={ldc} beta={beta}", flush=True)
+    assert "weight records in registers" in P.plan("int8", M, N, K)
+    q, sc = O.quant_rows(P.gen_activations(SEED, 1972 + M, M, K))
+    w = P.FvWeight(*_weight(K, N, 1982 + N), K, N)
+    C0 = np.random.default_rng(M).standard_normal((M, ldc)).astype(np.float32)
+    got = P.fvb_gemm_q8a("int8", q, sc, w, alpha=0.7, beta=beta, C0=C0)
+    monkeypatch.setenv("P2H_RECORDS_IN_REGISTERS", "0")
+    assert _bits_equal(got, P.fvb_gemm_q8a("int8", q, sc, w, alpha=0.7, beta=beta, C0=C0))
+    assert _bits_equal(got[:, N:], C0[:, N:])
+
+
 @pytest.mark.parametrize("M,K,N", [(2101, 128, 4112), (1025, 1024, 272), (1030, 1156, 16), (1100, 4096, 144)])
 def test_q8a_silu_large_tiles(M, K, N):
     """The int8w large-M tiles' SiLU (96 x 256 and 96 x 128, one and several fold blocks) with a cut last row tile and
     column tile: the bits of the GEMM followed by p2h_silu."""
     print(f"q8a silu large M={M} K={K} N={N} {P.plan('int8w', M, N, K)}", flush=True)
+    assert "weight records in registers" in P.plan("int8w", M, N, K)
     A = P.gen_activations(SEED, 1950 + M, M, K)
     q, sc = O.quant_rows(A)
     w = P.FvWeight(*_weight(K, N, 1960 + N), K, N)
@@ -734,6 +754,52 @@ def _expand64(signs, flags, lo, hi, N):
     code = ((signs[:, :, None] >> (2 * np.arange(4, dtype=np.uint8))) & 3).reshape(len(signs), N)
     flag = np.unpackbits(flags, axis=1, bitorder="little")[:, :N]
     return (code - 1.0) * np.where(flag != 0, lo + (hi - lo), lo).astype(np.float64)
+
+
+@pytest.mark.parametrize("K,lda", [(1024, 1024), (4096, 4096), (1000, 1000), (4004, 4004), (1024, 1025), (4096, 4097)])
+def test_exact_accuracy(monkeypatch, K, lda):
+    """The exact route against the product in 64 bits: relative error (2-norm) at most 5e-7 for every tile of gemm_xf
+    (rows staged, in registers by 16-byte loads and by elements; measured 1.2e-7 at K = 1024, 1.7e-7 at 4096) and for
+    gemm_xs. With the smallest of the three parts of a value left out it is about 1e-5."""
+    M, N = 2050, 2064
+    print(f"exact accuracy K={K} lda={lda} {P.plan('exact', M, N, K)}", flush=True)
+    planes = _weight(K, N, 983 + K)
+    w = P.FvWeight(*planes, K, N)
+    A = np.full((M, lda), np.nan, np.float32)
+    A[:, :K] = P.gen_activations(SEED, 984 + K, M, K)
+    ref = A[:, :K].astype(np.float64) @ _expand64(*planes, N)
+
+    def error(got, m):
+        return np.linalg.norm(got[:m].astype(np.float64) - ref[:m]) / np.linalg.norm(ref[:m])
+
+    assert error(P.fvb_gemm("exact", A, w), M) <= 5e-7   # gemm_xs where the rows allow 16-byte loads
+    for tile in (32, 64, 1616, 1632, 1664):
+        monkeypatch.setenv("P2H_XF_TILE", str(tile))
+        err = error(P.fvb_gemm("exact", A[:100], w), 100)
+        assert err <= 5e-7, f"tile {tile}: {err}"
+
+
+@pytest.mark.parametrize("M,K,N,lda,ldc", [(2050, 128, 2064, 132, 2064), (2050, 128, 2064, 128, 2067),
+                                            (2049, 100, 2064, 104, 2068), (1090, 1156, 4096, 1160, 4099)])
+def test_exact_many_rows_strides(monkeypatch, M, K, N, lda, ldc):
+    """gemm_xs with alpha, beta, strided A (NaN past K) and C (16-byte and element stores): gemm_xf's bits, the oracle
+    on a sample of rows, and columns past N as they were."""
+    print(f"exact many rows M={M} K={K} N={N} lda={lda} ldc={ldc}", flush=True)
+    assert "once per workgroup" in P.plan("exact", M, N, K)
+    signs, flags, lo, hi = _weight(K, N, 985 + K)
+    w = P.FvWeight(signs, flags, lo, hi, K, N)
+    A = np.full((M, lda), np.nan, np.float32)
+    A[:, :K] = P.gen_activations(SEED, 986 + M, M, K)
+    C0 = np.random.default_rng(M + K).standard_normal((M, ldc)).astype(np.float32)
+    rows = np.unique(np.concatenate([[0, M - 1], np.random.default_rng(K).choice(M, 16, replace=False)]))
+    for alpha, beta in [(1.0, 0.0), (0.5, 1.0), (-1.5, 0.3)]:
+        got = P.fvb_gemm("exact", A, w, alpha=alpha, beta=beta, C0=C0)
+        monkeypatch.setenv("P2H_XF_TILE", "64")
+        assert _bits_equal(got, P.fvb_gemm("exact", A, w, alpha=alpha, beta=beta, C0=C0)), f"alpha={alpha} beta={beta}"
+        monkeypatch.delenv("P2H_XF_TILE")
+        assert _bits_equal(got[:, N:], C0[:, N:])
+        _assert_exact(got[rows, :N], O.sgemm_fvb("exact", A[rows, :K].copy(), signs, flags, lo, hi, N, alpha=alpha,
+                                                 beta=beta, C0=C0[rows, :N].copy()))
 
 
 @pytest.mark.parametrize("M,K,N", [(40, 1024, 64), (37, 100, 80), (21, 1001, 48), (2050, 128, 2064), (2050, 100, 2064)])
