@@ -489,8 +489,9 @@ static P2hWeight *weight_new(int K, int N, bool copy_planes)
     return w;
 }
 
-/* Pinned words in which the weight kernels report to the host, one per upload under way (a copy back from device
- * memory cost an upload about 60 µs: 400 -> 467 for a 1024 x 3072 weight): as many as have ever been uploading at once, kept until the process ends. */
+/* Pinned words in which the weight kernels report to the host, one per upload under way (a copy back from device memory
+ * cost an upload about 60 µs: 400 -> 467 for a 1024 x 3072 weight): as many as have ever been uploading at once, kept
+ * until the process ends. */
 static std::mutex g_words_mu;
 static std::vector<uint32_t *> g_words;
 
@@ -1407,14 +1408,15 @@ ExactPlan exact_plan(int M, int N, int K, bool vec)
     const long long cus = g_cus > 0 ? g_cus : 256;
     auto tiles = [&](int bm, int bn) { return (long long)((N + bn - 1) / bn) * ((M + bm - 1) / bm); };
     const int forced = switch_of(g_sw.xf_tile);
-    /* many rows: where gemm_xs' tiles fill its two workgroups per CU at least once (M = 6000, 1024 -> 4096: 228 against
-     * 272 µs for gemm_xf's best tile; at 192 tiles, M = 375, 28.4 against 21.9) */
+    /* many rows: where gemm_xs' tiles fill its two workgroups per CU at least once. Against gemm_xf's best tile, by
+     * tiles: 384 1.01 to 1.08 of its time (320 1.17 to 1.26), 512 0.83 to 0.87 (M = 4096, 4096 -> 1024 176 -> 146 µs),
+     * 520 1.06 to 1.12 (its second round is nearly empty), 640 0.96 to 1.00, 752 and more 0.82 to 0.97. */
     if (forced == 0 && tiles(XsL::BM, XsL::BN) >= 2 * cus && K % 4 == 0 && K >= 64 && vec)
         return {true, XsL::BM, XsL::BN};
-    /* measured with the weights from HBM, the same bits for every tile: 16 × 16 while those fit the CUs in one round
-     * (M = 38, 4096 -> 1024: 10.7 against 11.4 µs for 16 × 32), 16 × 32 up to three per CU (M = 125, 1024 -> 1024: 5.4
-     * against 5.8 and 6.9 for 16 × 16 and 16 × 64; M = 375, 4096 -> 1024: 25.4 against 33.8 and 27.9), 16 × 64 up to
-     * six (M = 125, 1024 -> 4096: 9.9 against 10.7 and 10.1 for 16 × 32 and 32 × 64), else 32 × 64 */
+    /* measured with the weights in the caches: 16 × 16 while those fit the CUs in one round (M = 38, 4096 -> 1024: 7.8
+     * against 10.1 µs for 16 × 32), 16 × 32 up to three per CU (M = 200, 1024 -> 1024: 6.9 against 8.1 and 6.9 for
+     * 16 × 16 and 16 × 64; M = 375, 4096 -> 1024: 24.8 against 32.3 and 26.4), 16 × 64 up to six (M = 125, 1024 -> 4096:
+     * 9.0 against 10.2 and 9.7 for 16 × 32 and 32 × 64), else 32 × 64 */
     int bm = 16, bn = tiles(16, 16) <= cus ? 16 : tiles(16, 32) <= 3 * cus ? 32 : 64;
     if (bn == 64 && tiles(16, 64) > 6 * cus) bm = 32;
     if (forced == 32 || forced == 64) { bm = 32; bn = forced; }
@@ -1664,8 +1666,8 @@ static int launch_exact(int bkind, const p2k::ExactArgs &g0, hipStream_t s)
 }
 
 /* The exact five-value route on the matrix cores: gemm_xs for many rows, else gemm_xf (rows staged through LDS by
- * direct loads where K % 128 == 0 and the rows allow 16-byte loads; the same bits as the register path, which
- * P2H_XF_STAGED=0 selects). P2H_EXACT_CHAIN=1 selects gemm_exact instead, the reference's per-output fmaf chain bit for
+ * direct loads where K % 128 == 0 and the rows allow 16-byte loads; P2H_XF_STAGED=0 selects the register path): the same
+ * bits from each. P2H_EXACT_CHAIN=1 selects gemm_exact instead, the reference's per-output fmaf chain bit for
  * bit; P2H_XF_TILE forces gemm_xf and its tile. */
 }  // extern "C"
 

@@ -80,9 +80,9 @@ __device__ __forceinline__ uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel)
 /* ── per-column tables ─────────────────────────────────────────────────────────────────────────────────────── */
 
 /* clo[n] = clamp(lrintf(127·lo/hi), 0, 127), 0 when hi <= 0 (blas.c:1319-1326). The fold's other factors,
- * hi·(1/127) and hi − lo (blas.c:1327-1333), are made from lo and hi where they are used (c1_factor, c2_factor). */
-/* clo; and *odd = 1 where a column's lo or expanded hi is not finite or is 2^100 or more (the exact route's plane
- * kernels scale their sums by both, used or not). */
+ * hi·(1/127) and hi − lo (blas.c:1327-1333), are made from lo and hi where they are used (c1_factor, c2_factor).
+ * *odd = 1 where a column's lo or expanded hi is not finite or is 2^100 or more (the exact route's plane kernels scale
+ * their sums by both, used or not). */
 __global__ void fv_tables(int N, const float *__restrict__ lo, const float *__restrict__ hi, uint8_t *__restrict__ clo,
                           uint32_t *odd)
 {
@@ -2162,16 +2162,16 @@ __device__ __forceinline__ void fv_tile(const GemmArgs &g)
     }
 }
 
-/* The large-M int8w tiles with the weight records in registers (gemm_fv_rb, the production large-M kernel).
+/* The large-M tiles with the weight records in registers (gemm_fv_rb, the production large-M kernel).
  *  As fv_tile, except that each wave loads its own FN weight records of stage t + 1 straight into registers while
  *  stage t is computed (a wave is the only reader of its columns' records, so they need no LDS and no barrier), and
  *  decodes step 0 of stage t + 1 among stage t's step-1 MFMAs: a stage starts on MFMAs as soon as its first
  *  activation operands are read from LDS. Only the activation operands go through the LDS ring (direct loads, one
  *  barrier per stage). Against the records in LDS: M = 1500 11.3 against 12.4 µs, M = 4099 24.8 against 27.1,
- *  M = 6000 32.5 against 33.7 (1024 → 4096). The two-plane mode
- *  (K <= 1024) runs the 96 × 128 tile with two decoded operands and two sets of sums: M = 1501, 1024 → 3072 24 → 11 µs
- *  against the 128 × 128 tiles of fv_tile. Two workgroups per CU; the output is folded and staged as in
- *  fv_tile (per 1024-row block, in order; C staged through LDS as whole row segments at device scope). */
+ *  M = 6000 32.5 against 33.7 (1024 → 4096). The two-plane mode (K <= 1024) runs the 96 × 128 tile with two decoded
+ *  operands and two sets of sums: M = 1501, 1024 → 3072 24 → 11 µs against the 128 × 128 tiles of fv_tile. Two
+ *  workgroups per CU; the output is folded and staged as in fv_tile (per 1024-row block, in order; C staged through LDS
+ *  as whole row segments at device scope). */
 template <class G, int MODE, bool MULTI, bool ACT>
 __device__ __forceinline__ void fv_tile_rb(const GemmArgs &g)
 {
@@ -2941,7 +2941,8 @@ __global__ __launch_bounds__(256) void gemm_exact(ExactArgs g)
  * products to the row's finished sums, so that small values count in full, alone in a row or beside large ones. The
  * parts themselves may be denormal: these matrix instructions neither flush them nor the sums.
  *   Weights holding code 3 (twice the value, which no plane holds) or a lo or hi that is not finite or beyond 2^100
- * are left to gemm_exact (P2hWeight::planes). */
+ * are left to gemm_exact (P2hWeight::planes; M = 375, 1024 → 1024: 101 µs against 9). The five-value format has neither:
+ * its codes are 0 to 2 and its lo and hi are fp16 values. */
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
 /* The high halves of two floats as a dword of bf16: lo's in the low half. */
@@ -3043,14 +3044,15 @@ __device__ __forceinline__ v4f xs_complete(const ExactArgs &g, int m, int n, v4f
  * bf16 matrix cores (above), for up to a few hundred rows. The sum runs in a different order from the reference's
  * per-output fmaf chain (which gemm_exact keeps bit for bit), so outputs agree to fp32 rounding.
  * A workgroup owns a BM × BN tile and splits K among its NW waves, as gemm_fvs does, a wave to PPW pieces (XsCuts):
- * each wave streams its units' weight records (the 4-bit selectors of fv_repack4) and fp32 rows and splits and decodes both in registers;
- * lane l takes k = 16·(l / 16) .. + 15 of a 64-row step, which is the record's own order. The partial tiles
- * meet in LDS and are added in wave order.
+ * each wave streams its units' weight records (the 4-bit selectors of fv_repack4) and fp32 rows and splits and decodes
+ * both in registers; lane l takes k = 16·(l / 16) .. + 15 of a 64-row step, which is the record's own order. The
+ * partial tiles meet in LDS and are added in order of k.
  * The fp32 rows reach the lanes in one of two ways, with the same matrix instructions in the same order (the same
- * bits). Against the fp32 matrix cores (the same tiles, weights from HBM): M = 375, 1024 → 4096 34.0 → 21.9 µs,
- * 4096 → 1024 37.8 → 25.4, 1024 → 1024 13.0 → 9.3; M = 125, 1024 → 4096 13.9 → 9.9; M = 38, 4096 → 1024
- * 11.9 → 10.7. What bounds it now is the split itself (about six VALU operations per value and column tile) and, with
- * few waves per CU, the loads' latency:
+ * bits). Against the fp32 matrix cores (weights in the caches): M = 375, 1024 → 4096 31.6 → 20.6 µs, 4096 → 1024
+ * 38.8 → 24.8, 1024 → 1024 13.1 → 9.0; M = 125, 1024 → 4096 13.5 → 9.1; M = 38, 4096 → 1024 11.5 → 7.8. What bounds it
+ * now is the split itself (about six VALU operations per value and column tile: at M = 375 seven to nine VALU
+ * instructions of 4 cycles to a matrix one of 16, the matrix cores busy in 34 to 40 % of the cycles) and, with few
+ * waves per CU, the loads' latency:
  *   STAGED (K % 128 == 0 and VEC): each wave brings its 64-row K stages of the BM rows into its own LDS slot by
  *     direct loads of whole 256-byte row segments (four rows per instruction, 16-byte chunk c of row r stored at
  *     place c ^ (r % 16), so the operand reads below are free of bank conflicts); no barrier, each wave reads only its

@@ -22,10 +22,12 @@ struct XsGeo {
  * have 96 instructions a step for a thread's 16 split values. Waves are WM × WN over the tile, each FM row groups by
  * FN column groups; rows are two steps ahead in registers and one in the two-slot LDS ring (a barrier a step), records
  * a unit ahead in registers. At the end of each piece of K (XsCuts) the planes' sums are folded into running outputs,
- * which gives gemm_xf's bits. 64 × 128, two workgroups per
- * CU: M = 6000, 4096 → 1024 421 → 220 µs and 1024 → 4096 438 → 228, 1.37 PFLOP/s of bf16 products (a loop of nothing
- * but these matrix instructions runs at 1.7–1.8 on this card, power-bound); 48 × 128 was 228 / 230, 64 × 64 251 / 254,
- * and 96 × 128 spilled (289 / 300). */
+ * which gives gemm_xf's bits. 64 × 128, two workgroups per CU: M = 6000, 4096 → 1024 421 → 214 µs and 1024 → 4096
+ * 438 → 221 against the fp32 matrix cores, 1.41 PFLOP/s of bf16 products, where a loop of nothing but these matrix
+ * instructions reaches 1.7 on random operands and 2.0 on planes this sparse (power). Counters, launched back to back:
+ * the matrix cores are busy in 62 % of the cycles, at 1.9 GHz of the card's 2.4; three VALU instructions to a matrix
+ * one. Launched for longer than a few ms the clock falls further (281 µs in a replayed graph). Other tiles, with the
+ * sums folded every 512 rows: 48 × 128 1 to 4 % slower, 64 × 64 11 to 14 %, 96 × 128 spilled. */
 template <class G, bool TAIL>
 __global__ __launch_bounds__(G::NT, 2) void gemm_xs(ExactArgs g)
 {
