@@ -3146,6 +3146,14 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_xf(ExactArgs g)
             r[rb][i][0] = v.x; r[rb][i][1] = v.y; r[rb][i][2] = v.z; r[rb][i][3] = v.w;
         }
     };
+    /* PPW = 2: column n0 + lane's factors, held here: loads in the K loop would be waited for behind the rows' */
+    float lo2 = 0.0f, hi2 = 0.0f;
+    if (PPW == 2) {
+        const int n = min(n0 + (lane & (BN - 1)), N - 1);
+        lo2 = g.lo[n];
+        hi2 = 2.0f * __builtin_fmaf(1.0f, g.hi[n] - lo2, lo2);
+        lo2 *= 2.0f;
+    }
     /* this wave's sums of a piece: 2·lo and 2·hi (as the reference expands it) times the planes' */
     auto put_piece = [&](float *area) __attribute__((always_inline)) {
         int n_at = n0 + 4 * grp, at = wave * TILE + (lane & 15) * PITCH + 4 * grp;
@@ -3156,6 +3164,11 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_xf(ExactArgs g)
             float lo[4], hi[4];
 #pragma unroll
             for (int e = 0; e < 4; e++) {
+                if (PPW == 2) {
+                    lo[e] = __shfl(lo2, n_at - n0 + 16 * i + e);
+                    hi[e] = __shfl(hi2, n_at - n0 + 16 * i + e);
+                    continue;
+                }
                 lo[e] = g.lo[n + e];
                 hi[e] = 2.0f * __builtin_fmaf(1.0f, g.hi[n + e] - lo[e], lo[e]);
                 lo[e] *= 2.0f;
