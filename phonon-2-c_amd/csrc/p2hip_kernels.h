@@ -2934,11 +2934,11 @@ __global__ __launch_bounds__(256) void gemm_exact(ExactArgs g)
  * nearer to the 64-bit ones than the fp32 instructions' (relative error, K = 1024 and 4096): 1.2e-7 and 1.7e-7 against
  * 2.3e-7 and 4.5e-7.
  *   Outputs that come out infinite or NaN are summed again by a scalar chain of fmaf over the expanded weights
- * (xs_complete, slow): the planes' zeros make NaN of an infinity's parts, and sums of halves could overflow where those of
+ * (xs_finish, slow): the planes' zeros make NaN of an infinity's parts, and sums of halves could overflow where those of
  * the real products do not.
  *   bf16's smallest step is 2^-133, so of a value below 2^-110 the parts leave bits out: those of the third remainder
- * below that step. split8 notes that there are any (one operation in twelve of a pair) and xs_complete adds their
- * products to the row's finished sums, so that small values count in full, alone in a row or beside large ones. The
+ * below that step. split8 notes that there are any (one operation in twelve of a pair); a tile with such a row goes over
+ * them in a second pass (xs_low_bits), so that small values count in full, alone in a row or beside large ones. The
  * parts themselves may be denormal: these matrix instructions neither flush them nor the sums.
  *   Weights holding code 3 (twice the value, which no plane holds) or a lo or hi that is not finite or beyond 2^100
  * are left to gemm_exact (P2hWeight::planes; M = 375, 1024 → 1024: 101 µs against 9). The five-value format has neither:
@@ -3008,36 +3008,89 @@ __device__ __forceinline__ float left_out(float x)
     return t - cut_bf16(t);
 }
 
-/* The finished sums of outputs (m, n .. n + 3) made whole: finite ones take what the parts left out of a row with such
- * values (low); others are summed again, as one chain of fmaf over k with the weights as the reference expands them. One
- * loop for both, eight values at a time, since its code lies in every kernel's epilogue. */
-__device__ __forceinline__ v4f xs_complete(const ExactArgs &g, int m, int n, v4f sum, bool low)
+constexpr float kXsLift = 1267650600228229401496703205376.0f;   /* 2^100: lifts what is left out to normal values */
+
+/* What the parts leave out of the wave's rows, lifted, times the weights of units [u_begin, u_end): at most sixteen bits
+ * a value, so two parts. rows: the lane's row of each row group; b: the lane's records of each column group. Run for
+ * tiles with such a value only; to other rows it adds zeros. Alone, M = 375, 1024 → 4096 with such values in every row
+ * takes 75 µs against 26, M = 6000, 4096 → 1024 900 against 237; a chain of fmaf over them took 2.8 and 48 ms. */
+template <int FM, int FN>
+__device__ __forceinline__ void xs_low_bits(const float *const (&rows)[FM], const uint8_t *const (&b)[FN], int K,
+                                            int u_begin, int u_end, v4f (&accL)[FN][FM], v4f (&accH)[FN][FM])
+{
+    const int grp = (threadIdx.x & 63) >> 4;
+#pragma unroll 1
+    for (int q = 4 * u_begin; q < 4 * u_end; q++) {   /* a record's dwords: half q % 2 of step q / 2 % 2 of unit q / 4 */
+        const int k0 = 128 * (q >> 2) + 64 * ((q >> 1) & 1) + 16 * grp + 8 * (q & 1);
+        v8bf p[FM][3];
+#pragma unroll
+        for (int j = 0; j < FM; j++) {
+            float l[8];
+            uint32_t none = 0u;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float v = left_out(rows[j][min(k0 + e, K - 1)]) * kXsLift;
+                l[e] = k0 + e < K ? v : 0.0f;
+            }
+            split8(l, p[j], none);
+        }
+#pragma unroll
+        for (int i = 0; i < FN; i++) {
+            v8bf wl, wh;
+            decode_planes(*reinterpret_cast<const uint32_t *>(b[i] + (size_t)(q >> 2) * 1024 + 4 * (q & 3)), wl, wh);
+#pragma unroll
+            for (int s = 1; s >= 0; s--)
+#pragma unroll
+                for (int j = 0; j < FM; j++) {
+                    accL[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wl, p[j][s], accL[i][j], 0, 0, 0);
+                    accH[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wh, p[j][s], accH[i][j], 0, 0, 0);
+                }
+        }
+    }
+}
+
+/* The finished sums of outputs (m, n .. n + 3), which if infinite or NaN are summed again as one chain of fmaf over k
+ * with the weights as the reference expands them. A NaN in the row makes NaN of them all, found by a look over it. */
+__device__ __forceinline__ v4f xs_finish(const ExactArgs &g, int m, int n, v4f sum)
 {
     constexpr float top = 3.402823466e38f;
-    const bool again = !(__builtin_fabsf(sum[0]) <= top && __builtin_fabsf(sum[1]) <= top &&
-                         __builtin_fabsf(sum[2]) <= top && __builtin_fabsf(sum[3]) <= top);
-    if (!again && !low) return sum;
+    if (__builtin_fabsf(sum[0]) <= top && __builtin_fabsf(sum[1]) <= top && __builtin_fabsf(sum[2]) <= top &&
+        __builtin_fabsf(sum[3]) <= top)
+        return sum;
     const float *row = g.A + (size_t)m * g.lda;
-    v4f rest = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-    for (int k0 = 0; k0 < g.K; k0 += 8) {
-        float any = 0.0f;
+    for (int k = 0; k < g.K; k += 8) {
+        bool nan = false;
 #pragma unroll
-        for (int e = 0; e < 8; e++) any += __builtin_fabsf(left_out(row[min(k0 + e, g.K - 1)]));
-        if (!again && any == 0.0f) continue;
+        for (int e = 0; e < 8; e++) {
+            const float v = row[min(k + e, g.K - 1)];
+            nan |= v != v;
+        }
+        if (nan) {
+            const float v = __builtin_nanf("");
+            return v4f{v, v, v, v};
+        }
+    }
+    v4f chain = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 1
-        for (int k = k0; k < min(k0 + 8, g.K); k++) {
-            const float v = again ? row[k] : left_out(row[k]);
-            int shift;
-            const uint8_t *rb = g.rec + rec_quad_offset(g.units, k & ~3, n, shift) + (k & 3);
+    for (int k0 = 0; k0 < g.K; k0 += 4) {
+        int shift;
+        const uint8_t *rb = g.rec + rec_quad_offset(g.units, k0, n, shift);
+        uint32_t sel[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) sel[e] = *reinterpret_cast<const uint32_t *>(rb + 16 * e) >> shift;
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            if (k0 + b >= g.K) break;
+            const float a = row[k0 + b];
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const int sel = (rb[16 * e] >> shift) & 7;
-                const float lo = g.lo[n + e], w = __builtin_fmaf((float)(sel >> 2), g.hi[n + e] - lo, lo);
-                rest[e] = __builtin_fmaf(v, (float)((sel & 3) - 1) * w, rest[e]);
+                const float lo = g.lo[n + e], code = (float)((int)(sel[e] >> (8 * b) & 3u) - 1);
+                const float w = __builtin_fmaf((float)(sel[e] >> (8 * b + 2) & 1u), g.hi[n + e] - lo, lo);
+                chain[e] = __builtin_fmaf(a, code * w, chain[e]);
             }
         }
     }
-    return again ? rest : sum + rest;
+    return chain;
 }
 
 /* The exact-mode five-value GEMM (sgemm_fvb_exact, blas.c:929-987): C = beta·C + alpha·A·W with exact products on the
@@ -3061,7 +3114,7 @@ __device__ __forceinline__ v4f xs_complete(const ExactArgs &g, int m, int n, v4f
  *   else: loads into registers in the matrix-core layout, double-buffered.
  * VEC: K % 4 == 0, lda % 4 == 0 and A 16-byte aligned. */
 template <int FM, int FN, int NW, int PPW, bool VEC, bool STAGED = false>
-__global__ __launch_bounds__(64 * NW, 2) void gemm_xf(ExactArgs g)
+__global__ __launch_bounds__(64 * NW, STAGED && FM == 1 ? 4 : 2) void gemm_xf(ExactArgs g)
 {
     static_assert(!STAGED || VEC, "the staged rows are read as 16-byte chunks");
     static_assert(NW * PPW == 4 || NW * PPW == 8, "a quarter of K is one piece or two");
@@ -3299,20 +3352,51 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_xf(ExactArgs g)
     put_piece(part);
     __syncthreads();
 
-    constexpr int TPR = BN / 4, RPP = NT / TPR;
+    constexpr int TPR = BN / 4, RPP = NT / TPR, RPT = (BM + RPP - 1) / RPP;   /* RPT: rows per thread */
     const int cq = tid % TPR, n = n0 + 4 * cq;
-    if (n >= N) return;
-    for (int row = tid / TPR; row < BM; row += RPP) {
-        const int m = m0 + row;
-        if (m >= M) break;
+    auto add_pieces = [&](int t) __attribute__((always_inline)) {
         v4f sum = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int sg = 0; sg < NW; sg++) {
-            const int at = sg * TILE + row * PITCH + 4 * cq;
+            const int at = sg * TILE + min(tid / TPR + t * RPP, BM - 1) * PITCH + 4 * cq;
             if (PPW == 2) sum += *reinterpret_cast<const v4f *>(part1 + at);
             sum += *reinterpret_cast<const v4f *>(part + at);
         }
-        sum = xs_complete(g, m, n, sum, lowbits[row] != 0);
+        return sum;
+    };
+    v4f sums[RPT];
+#pragma unroll
+    for (int t = 0; t < RPT; t++) sums[t] = add_pieces(t);
+    if (__any(lowbits[min(lane, BM - 1)] != 0)) {   /* the same for every wave */
+        const float *rows[FM];
+        const uint8_t *recs[FN];
+        int ln = lane;
+        asm volatile("" : "+v"(ln));   /* the pointers are made here, not held through the K loop */
+#pragma unroll
+        for (int j = 0; j < FM; j++) rows[j] = g.A + (size_t)min(m0 + 16 * j + (ln & 15), M - 1) * g.lda;
+#pragma unroll
+        for (int i = 0; i < FN; i++) recs[i] = g.rec + (size_t)min((n0 >> 4) + i, N / 16 - 1) * units * 1024 + ln * 16;
+        __syncthreads();   /* the pieces are read */
+        if (PPW == 2) {
+            xs_low_bits<FM, FN>(rows, recs, K, w_begin, mid, accL, accH);
+            put_piece(part1);
+        }
+        xs_low_bits<FM, FN>(rows, recs, K, PPW == 2 ? mid : w_begin, w_end, accL, accH);
+        put_piece(part);
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < RPT; t++) {
+            const v4f low_sum = add_pieces(t);
+#pragma unroll
+            for (int e = 0; e < 4; e++) sums[t][e] = __builtin_fmaf(low_sum[e], 1.0f / kXsLift, sums[t][e]);
+        }
+    }
+    if (n >= N) return;
+#pragma unroll
+    for (int t = 0; t < RPT; t++) {
+        const int row = tid / TPR + t * RPP, m = m0 + row;
+        if (row >= BM || m >= M) break;
+        const v4f sum = xs_finish(g, m, n, sums[t]);
         float *cp = g.C + (size_t)m * g.ldc + n;
         if (n + 3 < N && (reinterpret_cast<uintptr_t>(cp) & 15) == 0) {   /* one 16-byte store */
             v4f c0 = v4f{0.0f, 0.0f, 0.0f, 0.0f};

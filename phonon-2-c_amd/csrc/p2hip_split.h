@@ -15,6 +15,7 @@ struct XsGeo {
     static constexpr int NO = (BM * 8 + NT - 1) / NT;       /* octets (8 consecutive k of a row) per thread and step */
     static constexpr int PITCH = BN + 4;                    /* floats per staged output row */
     static_assert(BM * PITCH * 4 <= 2 * STEP, "the outputs are staged in the ring");
+    static_assert(BM <= 64, "a lane per row's flag");
 };
 
 /* The exact route for many rows: products and parts as gemm_xf's, but a workgroup splits its rows once into LDS for
@@ -193,6 +194,30 @@ __global__ __launch_bounds__(G::NT, 2) void gemm_xs(ExactArgs g)
     for (int q = 0; q < NO; q++)
         if (has(q) && (low[q] & 0xffffu)) lowbits[(tid >> 3) + q * (NT / 8)] = 1;
     lds_barrier();   /* every wave is done with the ring: the outputs are staged in it */
+    if (__any(lowbits[lane % BM] != 0)) {   /* the same for every wave */
+        const float *rows[FM];
+#pragma unroll
+        for (int j = 0; j < FM; j++) rows[j] = g.A + (size_t)min(m0 + 16 * (wm * FM + j) + x, M - 1) * g.lda;
+        v4f sums[FN][FM];
+#pragma unroll
+        for (int i = 0; i < FN; i++)
+#pragma unroll
+            for (int j = 0; j < FM; j++) {
+                sums[i][j] = run[i][j];
+                run[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+        piece = cuts.half;
+        for (int u = 0; u < units; u += piece, piece = cuts.half < cuts.su ? cuts.su - piece : piece) {
+            xs_low_bits<FM, FN>(rows, b_src, K, u, min(units, u + piece), accL, accH);
+            fold();
+        }
+#pragma unroll
+        for (int i = 0; i < FN; i++)
+#pragma unroll
+            for (int j = 0; j < FM; j++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) run[i][j][e] = __builtin_fmaf(run[i][j][e], 1.0f / kXsLift, sums[i][j][e]);
+    }
     float *stg = reinterpret_cast<float *>(ring);
 #pragma unroll
     for (int i = 0; i < FN; i++)
@@ -208,8 +233,7 @@ __global__ __launch_bounds__(G::NT, 2) void gemm_xs(ExactArgs g)
     for (int row = tid / TPR; row < BM; row += RPP) {
         const int m = m0 + row;
         if (m >= M) break;
-        v4f sum = *reinterpret_cast<const v4f *>(stg + row * G::PITCH + 4 * cq);
-        sum = xs_complete(g, m, n, sum, lowbits[row] != 0);
+        const v4f sum = xs_finish(g, m, n, *reinterpret_cast<const v4f *>(stg + row * G::PITCH + 4 * cq));
         float *cp = g.C + (size_t)m * g.ldc + n;
         v4f c0 = v4f{0.0f, 0.0f, 0.0f, 0.0f};
         if (g.beta != 0.0f) {
