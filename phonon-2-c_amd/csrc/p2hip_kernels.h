@@ -3104,7 +3104,7 @@ __device__ __forceinline__ v4f xs_finish(const ExactArgs &g, int m, int n, v4f s
  * bits). Against the fp32 matrix cores (weights in the caches): M = 375, 1024 → 4096 31.6 → 20.6 µs, 4096 → 1024
  * 38.8 → 24.8, 1024 → 1024 13.1 → 9.0; M = 125, 1024 → 4096 13.5 → 9.1; M = 38, 4096 → 1024 11.5 → 7.8. What bounds it
  * now is the split itself (about six VALU operations per value and column tile: at M = 375 seven to nine VALU
- * instructions of 4 cycles to a matrix one of 16, the matrix cores busy in 34 to 40 % of the cycles) and, with few
+ * instructions of 4 cycles to a matrix one of 16, the matrix cores busy in 33 to 41 % of the cycles) and, with few
  * waves per CU, the loads' latency:
  *   STAGED (K % 128 == 0 and VEC): each wave brings its 64-row K stages of the BM rows into its own LDS slot by
  *     direct loads of whole 256-byte row segments (four rows per instruction, 16-byte chunk c of row r stored at

@@ -70,7 +70,7 @@ def _assert_exact(got, ref):
 @pytest.mark.parametrize("blocks", [2, 24])
 def test_exact_sweep_chain(monkeypatch, blocks):
     """The exact-mode sweep bench.py times (ExactChain: 9 linears per block at their real shapes, one graph per
-    window), on sampled rows. The fp32 matrix-core route: every linear within 1e-4 of the oracle's exact route
+    window), on sampled rows. The matrix-core route: every linear within 1e-4 of the oracle's exact route
     (blas.c:929-987) applied to the same input rows the device read (the chain's own earlier outputs), so each
     linear is held to the bar without the earlier linears' rounding compounding. The fmaf-chain route
     (P2H_EXACT_CHAIN=1 at capture): bit for bit the oracle's exact chain fed from its own outputs, every linear."""

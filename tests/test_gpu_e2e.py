@@ -5,7 +5,7 @@ GEMMs bound to libphonon2_gemm.so, against the same engine with its own GEMMs (e
 The encoder frames – the output of all 24 blocks' 216 five-value linears, the int8 subsampling and projector
 linears and everything between them – must be bit-identical (exact mode on the fmaf-chain route, P2H_EXACT_CHAIN=1,
 and the int8 modes), and the greedy TDT decoder must emit the same token ids; the reference CLI (main.c --tokens,
-through p2_engine_open / p2_transcribe) must print the same ids. Exact mode on the fp32 matrix cores sums in another
+through p2_engine_open / p2_transcribe) must print the same ids. Exact mode on the matrix cores sums in another
 order: its frames agree to fp32 rounding and its token ids are identical."""
 import numpy as np
 import pytest
@@ -40,7 +40,7 @@ def test_encoder_frames_and_tokens(fx, mode, reference):
 
 
 def test_encoder_exact_on_matrix_cores(fx):
-    """Exact mode on the fp32 matrix cores: the products are summed in another order than the reference's fmaf
+    """Exact mode on the matrix cores: the products are summed in another order than the reference's fmaf
     chain, so frames agree to fp32 rounding carried through 24 blocks, and the token ids are identical."""
     print("encdump_gpu (exact, matrix cores) vs encdump_cpu", flush=True)
     got, got_ids = run.encdump("gpu", "exact", fx + "/model", fx + "/a.wav", fx + "/gpu_exact_mfma.f32")
