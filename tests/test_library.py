@@ -105,8 +105,7 @@ def _kernel_metadata(so):
     """{kernel name: its metadata} of the gfx950 code objects inside a library built here: the AMDGPU metadata note
     (type 32, MessagePack) of every embedded ELF of machine 224."""
     import struct
-
-    import msgpack
+    msgpack = pytest.importorskip("msgpack")
     data, out, at = open(so, "rb").read(), {}, 0
     while (at := data.find(b"\x7fELF", at + 1)) > 0:
         if struct.unpack_from("<H", data, at + 18)[0] != 224:
